@@ -22,13 +22,17 @@
 // V is read as four token rows of D/16 contiguous elements (dims (D/16)n .. +D/16) and
 // transposed in registers with v_perm_b32 into the A operand of each of the D/16 M-tiles;
 // M-tile j, row r <-> dim (D/16)r + j. In the dense kernel all global loads are 16/8/4-byte
-// per lane and one K load instruction covers half of each of the tile's 16 rows. The paged
+// per lane and one K load instruction covers half of each of the tile's 16 rows. With fp32
+// q/k/v the same runs feed v_mfma_f32_16x16x4 (one dim, then one token per lane group and
+// instruction), with no permutes. The paged
 // kernel reads records whose V is stored transposed in groups of four tokens (PTile), so its
 // V operands arrive as 16-byte loads in MFMA order with no permutes.
 //
 // P is rounded to the K/V element type before the P.V product, as the reference does
 // (streaming_attention.py:178, :347, :428).
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "pgr_common.h"
 #include "pgr_kernels.h"
@@ -81,81 +85,117 @@ __device__ __forceinline__ float wave_sum_g(float x) {
   return x + __shfl_xor(x, 32);
 }
 
-// Registers of one 16-token tile held by one lane.
-template <int D>
-struct Tile {
-  static_assert(D == 32 || D == 64 || D == 128, "head_dim must be 32, 64 or 128");
-  static constexpr int KV4 = D / 32;  // u32x4 of K per lane (D/4 elements)
-  static constexpr int VW = D / 32;   // dwords of V per token row per lane (D/16 elements)
-  u32x4 k[KV4];
-  uint32_t v[4][VW];
+// fp32 q/k/v (the dense operator kernels only): one dword per operand and lane.
+struct F32 {
+  static __device__ __forceinline__ f32x4 mma(uint32_t a, uint32_t b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b), c, 0, 0,
+                                                0);
+  }
 };
 
-// K row `row` of the tile at `tile_k` (row stride D elements): elements (D/4)g .. +D/4.
-template <int D>
-__device__ __forceinline__ void load_k(Tile<D>& t, const uint16_t* tile_k, int row, int g) {
-  const u32x4* p = reinterpret_cast<const u32x4*>(tile_k + (size_t)row * D + (D / 4) * g);
-#pragma unroll
-  for (int i = 0; i < Tile<D>::KV4; ++i) t.k[i] = p[i];
-}
+// Dense operands are only as aligned as their elements (a caller's view may start anywhere):
+// the vector types say so, and the loads stay one instruction each.
+typedef uint32_t u32_e __attribute__((aligned(2)));
+typedef uint32_t u32x2_e __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t u32x4_e __attribute__((ext_vector_type(4), aligned(2)));
 
-// V rows rows[0..3] at `tile_v`: elements (D/16)n .. +D/16 of each.
-template <int D>
-__device__ __forceinline__ void load_v(Tile<D>& t, const uint16_t* tile_v, const int (&rows)[4], int n) {
+// Registers of one 16-token tile held by one lane: D/4 elements of K row n, and D/16 elements
+// of each of four V rows (at 16-bit head dim 16 a single element, in the low half).
+template <class Ty, int D>
+struct Tile {
+  static_assert(D >= 16 && D <= 256, "head_dim must be 16 to 256 (8 runs as a padded 16)");
+  static constexpr int ES = std::is_same<Ty, F32>::value ? 4 : 2;  // element bytes
+  static constexpr int KD = D * ES / 16;                          // dwords of K
+  static constexpr int VD = D * ES >= 64 ? D * ES / 64 : 1;       // dwords of each V row
+  static constexpr bool kHalfV = D * ES < 64;                     // one 16-bit element per V row
+  uint32_t k[KD];
+  uint32_t v[4][VD];
+};
+
+template <int N>
+__device__ __forceinline__ void load_dwords(uint32_t (&r)[N], const void* src) {
+  const char* p = static_cast<const char*>(src);
+  if constexpr (N % 4 == 0) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint16_t* p = tile_v + (size_t)rows[i] * D + (D / 16) * n;
-    if constexpr (D == 32) {
-      t.v[i][0] = *reinterpret_cast<const uint32_t*>(p);
-    } else if constexpr (D == 64) {
-      u32x2 x = *reinterpret_cast<const u32x2*>(p);
-      t.v[i][0] = x.x;
-      t.v[i][1] = x.y;
-    } else {
-      u32x4 x = *reinterpret_cast<const u32x4*>(p);
-      t.v[i][0] = x.x;
-      t.v[i][1] = x.y;
-      t.v[i][2] = x.z;
-      t.v[i][3] = x.w;
+    for (int i = 0; i < N / 4; ++i) {
+      const u32x4 x = *reinterpret_cast<const u32x4_e*>(p + 16 * i);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) r[4 * i + c] = x[c];
     }
+  } else if constexpr (N == 2) {
+    const u32x2 x = *reinterpret_cast<const u32x2_e*>(p);
+    r[0] = x.x;
+    r[1] = x.y;
+  } else {
+    static_assert(N == 1, "1, 2 or a multiple of 4 dwords");
+    r[0] = *reinterpret_cast<const u32_e*>(p);
   }
 }
 
-template <int D>
-__device__ __forceinline__ void zero_v_row(Tile<D>& t, int i) {
+// The lane's run of row `row` (elements (D/4)g .. +D/4) of an array with DR elements per row.
+// DR < D: head dim 8 in the 16-wide layout, whose lane groups g >= 2 hold zeros.
+template <class Ty, int D, int DR, int N>
+__device__ __forceinline__ void load_run(uint32_t (&r)[N], const char* rows, size_t row, int g) {
+  if constexpr (DR < D) {
 #pragma unroll
-  for (int w = 0; w < Tile<D>::VW; ++w) t.v[i][w] = 0u;
+    for (int i = 0; i < N; ++i) r[i] = 0u;
+    if (g >= 2) return;
+  }
+  load_dwords(r, rows + (row * DR + (size_t)(D / 4) * g) * Tile<Ty, D>::ES);
 }
 
-// K operand (A of S^T) for contraction chunk c: dwords 2c, 2c+1 of the lane's K run.
-template <int D>
-__device__ __forceinline__ u32x2 k_chunk(const u32x4 (&k)[D / 32], int c) {
-  const u32x4 q = k[c >> 1];
-  return (c & 1) ? u32x2{q.z, q.w} : u32x2{q.x, q.y};
+// V rows rows[0..3] at `tile_v`: elements (D/16)n .. +D/16 of each.
+template <class Ty, int D, int DR>
+__device__ __forceinline__ void load_v(Tile<Ty, D>& t, const char* tile_v, const int (&rows)[4], int n) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (DR < D) {
+      t.v[i][0] = 0u;
+      if (n >= DR) continue;
+    }
+    const char* p = tile_v + ((size_t)rows[i] * DR + (D / 16) * n) * Tile<Ty, D>::ES;
+    if constexpr (Tile<Ty, D>::kHalfV)
+      t.v[i][0] = *reinterpret_cast<const uint16_t*>(p);
+    else
+      load_dwords(t.v[i], p);
+  }
 }
 
 // V^T operand (A of O^T) for M-tile j: element j of each of the four token rows.
-template <int D>
-__device__ __forceinline__ u32x2 v_tile(const uint32_t (&v)[4][D / 32], int j) {
+template <int VD>
+__device__ __forceinline__ u32x2 v_tile(const uint32_t (&v)[4][VD], int j) {
   const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
   const int w = j >> 1;
   return u32x2{__builtin_amdgcn_perm(v[1][w], v[0][w], sel), __builtin_amdgcn_perm(v[3][w], v[2][w], sel)};
 }
 
-// S^T tile of 16 tokens x 16 heads.
-template <class Ty, int D>
-__device__ __forceinline__ f32x4 qk_tile(const u32x4 (&k)[D / 32], const u32x4 (&q)[D / 32]) {
-  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+// Dwords [0, N) of the S^T contraction: k and q hold the same dims of a K row and a query.
+template <class Ty, int N>
+__device__ __forceinline__ f32x4 qk_dwords(const uint32_t* k, const uint32_t* q, f32x4 s) {
+  if constexpr (std::is_same<Ty, F32>::value) {
 #pragma unroll
-  for (int c = 0; c < D / 16; ++c) s = Ty::mma(k_chunk<D>(k, c), k_chunk<D>(q, c), s);
+    for (int c = 0; c < N; ++c) s = Ty::mma(k[c], q[c], s);
+  } else {
+#pragma unroll
+    for (int c = 0; c < N; c += 2) s = Ty::mma(u32x2{k[c], k[c + 1]}, u32x2{q[c], q[c + 1]}, s);
+  }
   return s;
 }
 
+// O^T[D x 16 heads] += V^T . P^T. 16-bit: P rounded to the K/V type, one product per M-tile;
+// fp32: one product per token of the lane's four and M-tile, P as it is.
 template <class Ty, int D>
-__device__ __forceinline__ void pv_tile(f32x4 (&acc)[D / 16], const Tile<D>& t, const float (&p)[4]) {
-  const u32x2 pb = {Ty::pack(p[0], p[1]), Ty::pack(p[2], p[3])};
+__device__ __forceinline__ void pv_tile(f32x4 (&acc)[D / 16], const Tile<Ty, D>& t, const float (&p)[4]) {
+  if constexpr (std::is_same<Ty, F32>::value) {
 #pragma unroll
-  for (int j = 0; j < D / 16; ++j) acc[j] = Ty::mma(v_tile<D>(t.v, j), pb, acc[j]);
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < D / 16; ++j) acc[j] = Ty::mma(t.v[i][j], __builtin_bit_cast(uint32_t, p[i]), acc[j]);
+  } else {
+    const u32x2 pb = {Ty::pack(p[0], p[1]), Ty::pack(p[2], p[3])};
+#pragma unroll
+    for (int j = 0; j < D / 16; ++j) acc[j] = Ty::mma(v_tile(t.v, j), pb, acc[j]);
+  }
 }
 
 // Scale + optional softcap of one raw score (streaming_attention.py:158-160).
@@ -169,18 +209,6 @@ __device__ __forceinline__ float transform_score(float s, float scale, float sof
 template <int D>
 __device__ __forceinline__ int acc_dim(int g, int i, int j) {
   return (D / 4) * g + (D / 16) * i + j;
-}
-
-// Q^T operand for query head (row index `qrow` of a [rows, D] array); zero for padding heads.
-template <int D>
-__device__ __forceinline__ void load_q(u32x4 (&q)[D / 32], const uint16_t* qptr, bool real, int g) {
-#pragma unroll
-  for (int i = 0; i < D / 32; ++i) q[i] = u32x4{0u, 0u, 0u, 0u};
-  if (real) {
-    const u32x4* p = reinterpret_cast<const u32x4*>(qptr + (D / 4) * g);
-#pragma unroll
-    for (int i = 0; i < D / 32; ++i) q[i] = p[i];
-  }
 }
 
 template <bool kLog2>
@@ -202,7 +230,8 @@ struct MergeSmem {
 };
 
 // kLog2: (m, scores) are in log2 units and the weights are exp2(m_w - m); otherwise e-based.
-template <int D, bool kFold, bool kWithAcc, bool kLog2 = false>
+// DR: the head dim stored per head (8 for a padded 16).
+template <int D, bool kFold, bool kWithAcc, bool kLog2 = false, int DR = D>
 __device__ __forceinline__ void wg_merge_store(MergeSmem<D>& sm, int wave, int g, int n, float m_run, float l_lane,
                                                const f32x4 (&acc)[D / 16], int n_rep, float* pm, float* pl,
                                                float* pacc) {
@@ -235,8 +264,8 @@ __device__ __forceinline__ void wg_merge_store(MergeSmem<D>& sm, int wave, int g
     }
   }
   if constexpr (kWithAcc) {
-    for (int idx = tid; idx < n_rep * D; idx += kWaves * kWaveSize) {
-      const int r = idx / D, d = idx - r * D;
+    for (int idx = tid; idx < n_rep * DR; idx += kWaves * kWaveSize) {
+      const int r = idx / DR, d = idx - r * DR;
       float a = 0.f;
       if constexpr (kFold) {
         float mw = kNegInf;
@@ -262,9 +291,9 @@ __device__ __forceinline__ void wg_merge_store(MergeSmem<D>& sm, int wave, int g
 enum DenseMode : int { kModeFold = 0, kModeStats = 1, kModeAccumulate = 2, kModeFoldFixed = 3 };
 
 struct DenseArgs {
-  const uint16_t* q;
-  const uint16_t* k;
-  const uint16_t* v;
+  const char* q;          // elements of the kernel's type
+  const char* k;
+  const char* v;
   const int32_t* valid;   // [B, Tc] or null (all valid)
   const int32_t* active;  // [B] or null (all active)
   const float* m_in;      // FIXED modes: final m [B, Hq]
@@ -278,11 +307,28 @@ struct DenseArgs {
   float scale, softcap;
 };
 
-template <class Ty, int D, int kMode>
+// Memory-bound at every type and head dim: K and V are read once, in 16-byte pieces where a
+// lane's run is that long, and both products run on the matrix cores (on the VALU, with a K row
+// per lane, fp32 and the 16-bit head dims 8, 16 and 256 ran at 0.2-1.0 TB/s). Launches back to
+// back over chunk copies beyond the MALL, VALU kernel -> this one: bf16 D 256 (8/1 heads, batch
+// 8, 8192 tokens, 67 MB) 98.1 -> 16.6 us; fp32 D 64 (32/4, batch 2, 8001, 33 MB) 59.3 -> 8.5;
+// fp32 D 128 (28/4, batch 1, 32768, 134 MB) 141 -> 28.1; fp16 D 256 (16/8, batch 8, 16384,
+// 1.07 GB) 1085 -> 186 (5.8 TB/s).
+//
+// Below 64 dwords per lane and tile, two tiles per wave are in flight (double-buffered
+// registers). From 64 on (16-bit D 256, fp32 D 128) the tile is single-buffered in halves: the
+// next K is loaded under the softmax and P.V, the next V under the next scores. That needs half
+// the registers, so two waves per SIMD instead of one: 16.6 against 18.5 us at bf16 D 256, 28.1
+// against 27.7 at fp32 D 128. At fp32 D 256 (128 dwords) q comes from LDS as well.
+template <class Ty, int D, int DR, int kMode>
 __global__ __launch_bounds__(256) void dense_attn_kernel(DenseArgs a) {
+  using T = Tile<Ty, D>;
   constexpr bool kFold = (kMode == kModeFold || kMode == kModeStats);
   constexpr bool kWithV = (kMode != kModeStats);
   constexpr bool kMass = (kMode == kModeAccumulate);
+  constexpr bool kSingle = T::KD + 4 * T::VD >= 64;
+  constexpr bool kQLds = T::KD + 4 * T::VD > 64;
+  constexpr int kQStride = D + 4;  // LDS q rows (kQLds): 16 bytes apart in banks
   __shared__ MergeSmem<D> sm;
 
   const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
@@ -292,9 +338,9 @@ __global__ __launch_bounds__(256) void dense_attn_kernel(DenseArgs a) {
   const bool real = n < a.n_rep;
   const int qh = h * a.n_rep + (real ? n : 0);
 
-  const size_t kv_base = ((size_t)b * a.hkv + h) * (size_t)a.tc * D;
-  const uint16_t* kp = a.k + kv_base;
-  const uint16_t* vp = a.v + kv_base;
+  const size_t kv_base = ((size_t)b * a.hkv + h) * (size_t)a.tc * DR * T::ES;
+  const char* kp = a.k + kv_base;
+  const char* vp = kWithV ? a.v + kv_base : nullptr;
 
   const int t_begin = split * kWaves * a.wave_tokens + wave * a.wave_tokens;
   const int t_end = min(t_begin + a.wave_tokens, a.tc);
@@ -303,33 +349,55 @@ __global__ __launch_bounds__(256) void dense_attn_kernel(DenseArgs a) {
 
   // Tile ti's K and V (rows past the chunk clamped to its last row, then masked) and which of
   // the lane's four V rows are valid tokens.
-  auto fetch = [&](Tile<D>& t, bool (&ok)[4], int ti) {
-    const int t0 = t_begin + ti * 16;
-    load_k<D>(t, kp, min(t0 + n, a.tc - 1), g);
+  auto fetch_k = [&](T& t, int ti) {
+    load_run<Ty, D, DR>(t.k, kp, (size_t)min(t_begin + ti * 16 + n, a.tc - 1), g);
+  };
+  auto fetch_v = [&](T& t, bool (&ok)[4], int ti) {
     int rows[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int tok = t0 + 4 * g + i;
+      const int tok = t_begin + ti * 16 + 4 * g + i;
       ok[i] = tok < t_end;
       if (ok[i] && a.valid != nullptr) ok[i] = a.valid[(size_t)b * a.tc + tok] != 0;
       rows[i] = min(tok, a.tc - 1);
     }
-    if constexpr (kWithV) load_v<D>(t, vp, rows, n);
+    if constexpr (kWithV) load_v<Ty, D, DR>(t, vp, rows, n);
+  };
+  auto fetch = [&](T& t, bool (&ok)[4], int ti) {
+    fetch_k(t, ti);
+    fetch_v(t, ok, ti);
   };
 
-  Tile<D> ta, tb;
-  bool oka[4], okb[4];
+  T ta;
+  bool oka[4];
   if (tiles > 0) fetch(ta, oka, 0);  // the first tile's loads go out before the query's
 
-  u32x4 q[D / 32];
-  load_q<D>(q, a.q + ((size_t)b * a.hq + qh) * D, real, g);
+  const char* q_row = a.q;
+  const size_t q_idx = (size_t)b * a.hq + qh;
+  uint32_t q[kQLds ? 1 : T::KD];
+  float* q_s = &sm.acc[0][0][0];  // kQLds: [kMaxRep][kQStride], until the workgroup merge
+  if constexpr (kQLds) {
+    static_assert(std::is_same<Ty, F32>::value, "q of one dword per element");
+    static_assert(kMaxRep * kQStride <= kWaves * kMaxRep * (D + 1), "q fits the merge buffer");
+    const uint32_t* qsrc = reinterpret_cast<const uint32_t*>(q_row) + ((size_t)b * a.hq + (size_t)h * a.n_rep) * D;
+    for (int i = threadIdx.x; i < kMaxRep * D; i += kWaves * kWaveSize) {
+      const int r = i / D;
+      const uint32_t x = r < a.n_rep ? *reinterpret_cast<const u32_e*>(qsrc + i) : 0u;
+      q_s[r * kQStride + (i - r * D)] = __builtin_bit_cast(float, x);
+    }
+    __syncthreads();
+  } else {
+#pragma unroll
+    for (int i = 0; i < T::KD; ++i) q[i] = 0u;
+    if (real) load_run<Ty, D, DR>(q, q_row, q_idx, g);
+  }
 
   float m_run = kNegInf, l_run = 0.f;
   float m_fix = 0.f, l_fix = 1.f;
   if constexpr (!kFold) {
     if (real) {
-      m_fix = a.m_in[(size_t)b * a.hq + qh];
-      l_fix = a.l_in[(size_t)b * a.hq + qh];
+      m_fix = a.m_in[q_idx];
+      l_fix = a.l_in[q_idx];
     }
   }
   f32x4 acc[D / 16];
@@ -337,14 +405,31 @@ __global__ __launch_bounds__(256) void dense_attn_kernel(DenseArgs a) {
   for (int j = 0; j < D / 16; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   float blk = 0.f;
 
-  auto process = [&](Tile<D>& t, const bool (&ok)[4], int ti) {
-    const int t0 = t_begin + ti * 16;
+  auto scores = [&](const T& t) {
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (kQLds) {
+      const u32x4* ql = reinterpret_cast<const u32x4*>(q_s + n * kQStride + (D / 4) * g);
+#pragma unroll
+      for (int c = 0; c < T::KD / 4; ++c) {
+        const u32x4 qv = ql[c];
+        const uint32_t qc[4] = {qv.x, qv.y, qv.z, qv.w};
+        s = qk_dwords<Ty, 4>(t.k + 4 * c, qc, s);
+      }
+      return s;
+    } else {
+      return qk_dwords<Ty, T::KD>(t.k, q, s);
+    }
+  };
+
+  auto fold = [&](T& t, const f32x4& s4, const bool (&ok)[4], int ti) {
     if constexpr (kWithV) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (!ok[i]) zero_v_row<D>(t, i);
+        if (!ok[i]) {
+#pragma unroll
+          for (int w = 0; w < T::VD; ++w) t.v[i][w] = 0u;
+        }
     }
-    const f32x4 s4 = qk_tile<Ty, D>(t.k, q);
     float s[4], p[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) s[i] = ok[i] ? transform_score(s4[i], a.scale, a.softcap) : kNegInf;
@@ -372,8 +457,8 @@ __global__ __launch_bounds__(256) void dense_attn_kernel(DenseArgs a) {
         if ((ti + 1) % tiles_per_block == 0 || ti + 1 == tiles) {
           const float bs = wave_sum_g(blk);
           if (g == 0 && real) {
-            const int j = t0 / a.tokens_per_block;
-            a.block_mass[((size_t)b * a.hq + qh) * a.max_blocks + a.block_id_offset + j] = bs / l_fix;
+            const int j = (t_begin + ti * 16) / a.tokens_per_block;
+            a.block_mass[q_idx * a.max_blocks + a.block_id_offset + j] = bs / l_fix;
           }
           blk = 0.f;
         }
@@ -381,241 +466,40 @@ __global__ __launch_bounds__(256) void dense_attn_kernel(DenseArgs a) {
     }
   };
 
-  // Two tiles per wave in flight: the next tile's loads are issued before the current tile is
-  // folded. Unconditional in the loop (a conditional fetch lets the compiler drain the load
-  // queue every iteration); the last one or two tiles are folded after it.
-  int ti = 0;
-  for (; ti + 2 < tiles; ti += 2) {
-    fetch(tb, okb, ti + 1);
-    process(ta, oka, ti);
-    fetch(ta, oka, ti + 2);
-    process(tb, okb, ti + 1);
-  }
-  if (ti + 1 < tiles) {
-    fetch(tb, okb, ti + 1);
-    process(ta, oka, ti);
-    process(tb, okb, ti + 1);
-  } else if (ti < tiles) {
-    process(ta, oka, ti);
+  if constexpr (kSingle) {
+    for (int ti = 0; ti + 1 < tiles; ++ti) {
+      const f32x4 s4 = scores(ta);
+      fetch_k(ta, ti + 1);
+      fold(ta, s4, oka, ti);
+      fetch_v(ta, oka, ti + 1);
+    }
+    if (tiles > 0) fold(ta, scores(ta), oka, tiles - 1);
+    if constexpr (kQLds) __syncthreads();  // q_s and the merge share LDS
+  } else {
+    // The next tile's loads are issued before the current tile is folded. Unconditional in the
+    // loop (a conditional fetch lets the compiler drain the load queue every iteration); the
+    // last one or two tiles are folded after it.
+    T tb;
+    bool okb[4];
+    int ti = 0;
+    for (; ti + 2 < tiles; ti += 2) {
+      fetch(tb, okb, ti + 1);
+      fold(ta, scores(ta), oka, ti);
+      fetch(ta, oka, ti + 2);
+      fold(tb, scores(tb), okb, ti + 1);
+    }
+    if (ti + 1 < tiles) {
+      fetch(tb, okb, ti + 1);
+      fold(ta, scores(ta), oka, ti);
+      fold(tb, scores(tb), okb, ti + 1);
+    } else if (ti < tiles) {
+      fold(ta, scores(ta), oka, ti);
+    }
   }
 
   const size_t slot = ((size_t)b * a.hkv + h) * a.n_split + split;
-  wg_merge_store<D, kFold, kWithV>(sm, wave, g, n, m_run, l_run, acc, a.n_rep, a.pm + slot * a.n_rep,
-                                   a.pl + slot * a.n_rep, a.pacc + slot * a.n_rep * D);
-}
-
-// l of head r from a per-head register array, with r a per-lane value (no dynamic indexing).
-template <int N>
-__device__ __forceinline__ float l_run_at(const float (&l)[N], int r) {
-  float x = 0.f;
-#pragma unroll
-  for (int q = 0; q < N; ++q)
-    if (q == r) x = l[q];
-  return x;
-}
-
-// ---------------------------------------------------------------------------------------
-// Generic dense chunk kernel: the operator API for the cases the MFMA kernel above does not
-// take -- fp32 q/k/v (any head dim) and 16-bit head dims 8, 16 and 256. The reference pads
-// Q and K with zero columns up to 16 when head_dim < 16 (streaming_attention.py:56-66,
-// :125-133) so that tl.dot applies; zero columns add nothing to a dot product, and this
-// kernel computes the unpadded dot products directly on the VALU.
-//
-// One wave per workgroup, grid (n_split, Hkv, B); the wave folds `wave_tokens` consecutive
-// tokens in tiles of 64, with the same partial layout and e-based (m, l) as
-// dense_attn_kernel, so dense_merge_kernel combines either. Per tile:
-//   1. scores: lane t takes token t0 + t and all n_rep query heads (q in LDS);
-//   2. softmax: per head, a wave max / sum; P (rounded to the K/V type before P.V, as
-//      streaming_attention.py:178 does) goes to LDS;
-//   3. P.V: lane (g, c) takes head dims c, c + 64, ... of tokens g, g + G, ... (G = 64 / min(D, 64)),
-//      so each V row is read by consecutive lanes; the token groups are summed at the end.
-constexpr int kGenTile = 64;
-
-template <class Ty>
-struct GenElem {  // 16-bit K/V/q elements
-  typedef uint16_t T;
-  static __device__ __forceinline__ float ld(const T* p) { return Ty::to_f(*p); }
-  static __device__ __forceinline__ float round_p(float p) { return Ty::to_f(Ty::cvt(p)); }
-};
-struct F32Elem {
-  typedef float T;
-  static __device__ __forceinline__ float ld(const T* p) { return *p; }
-  static __device__ __forceinline__ float round_p(float p) { return p; }
-};
-
-__device__ __forceinline__ float wave_max64(float x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x = fmaxf(x, __shfl_xor(x, o));
-  return x;
-}
-__device__ __forceinline__ float wave_sum64(float x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-  return x;
-}
-
-template <class E, int D, int kMode>
-__global__ __launch_bounds__(64) void dense_generic_kernel(DenseArgs a) {
-  constexpr bool kFold = (kMode == kModeFold || kMode == kModeStats);
-  constexpr bool kWithV = (kMode != kModeStats);
-  constexpr bool kMass = (kMode == kModeAccumulate);
-  constexpr int DL = D < 64 ? D : 64;  // lanes per token group in the P.V pass
-  constexpr int G = 64 / DL;           // token groups
-  constexpr int DPL = D / DL;          // head dims per lane
-  typedef typename E::T T;
-  __shared__ float q_s[kMaxRep][D];
-  __shared__ float p_s[kMaxRep][kGenTile];    // P rounded for P.V
-  __shared__ float praw_s[kMaxRep][kGenTile];  // P unrounded, for the block mass
-  __shared__ float alpha_s[kMaxRep];
-
-  const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  if (a.active != nullptr && a.active[b] == 0) return;  // whole workgroup: uniform exit
-  const int lane = threadIdx.x;
-  const int n_rep = a.n_rep;
-  const size_t kv_base = ((size_t)b * a.hkv + h) * (size_t)a.tc * D;
-  const T* kp = reinterpret_cast<const T*>(a.k) + kv_base;
-  const T* vp = reinterpret_cast<const T*>(a.v) + kv_base;
-  const T* qp = reinterpret_cast<const T*>(a.q) + ((size_t)b * a.hq + (size_t)h * n_rep) * D;
-  for (int i = lane; i < kMaxRep * D; i += 64) {
-    const int r = i / D;
-    q_s[r][i - r * D] = r < n_rep ? E::ld(qp + i) : 0.f;
-  }
-  // Running (m, l) per head: uniform values, kept in registers of every lane.
-  float m_run[kMaxRep], l_run[kMaxRep], blk[kMaxRep];
-#pragma unroll
-  for (int r = 0; r < kMaxRep; ++r) {
-    m_run[r] = kNegInf;
-    l_run[r] = 0.f;
-    blk[r] = 0.f;
-    if constexpr (!kFold) {
-      if (r < n_rep) {
-        m_run[r] = a.m_in[(size_t)b * a.hq + h * n_rep + r];
-        l_run[r] = a.l_in[(size_t)b * a.hq + h * n_rep + r];
-      }
-    }
-  }
-  float acc[kMaxRep][DPL];
-#pragma unroll
-  for (int r = 0; r < kMaxRep; ++r)
-#pragma unroll
-    for (int j = 0; j < DPL; ++j) acc[r][j] = 0.f;
-  __syncthreads();
-
-  const int t_begin = split * a.wave_tokens;
-  const int t_end = min(t_begin + a.wave_tokens, a.tc);
-  const int grp = lane / DL, col = lane - grp * DL;
-  for (int t0 = t_begin; t0 < t_end; t0 += kGenTile) {
-    // 1. Scores of token t0 + lane for every head.
-    const int t = t0 + lane;
-    bool ok = t < t_end;
-    if (ok && a.valid != nullptr) ok = a.valid[(size_t)b * a.tc + t] != 0;
-    float s[kMaxRep];
-#pragma unroll
-    for (int r = 0; r < kMaxRep; ++r) s[r] = 0.f;
-    if (ok) {
-      const T* krow = kp + (size_t)t * D;
-      for (int d = 0; d < D; ++d) {
-        const float kd = E::ld(krow + d);
-#pragma unroll
-        for (int r = 0; r < kMaxRep; ++r) s[r] += q_s[r][d] * kd;
-      }
-    }
-    // 2. Softmax weights per head.
-#pragma unroll
-    for (int r = 0; r < kMaxRep; ++r) {
-      if (r >= n_rep) continue;  // uniform
-      const float x = ok ? transform_score(s[r], a.scale, a.softcap) : kNegInf;
-      float p;
-      if constexpr (kFold) {
-        const float m_new = fmaxf(m_run[r], wave_max64(x));
-        const bool empty = m_new == kNegInf;
-        const float alpha = empty ? 0.f : __expf(m_run[r] - m_new);
-        p = (empty || !ok) ? 0.f : __expf(x - m_new);
-        l_run[r] = l_run[r] * alpha + wave_sum64(p);
-        m_run[r] = m_new;
-        if (lane == 0) alpha_s[r] = alpha;
-      } else {
-        p = ok ? __expf(x - m_run[r]) : 0.f;
-      }
-      p_s[r][lane] = E::round_p(p);
-      if constexpr (kMass) praw_s[r][lane] = p;
-    }
-    __syncthreads();
-    // 3. P.V over this tile.
-    if constexpr (kWithV) {
-      if constexpr (kFold) {
-#pragma unroll
-        for (int r = 0; r < kMaxRep; ++r) {
-          if (r >= n_rep) continue;
-          const float al = alpha_s[r];
-#pragma unroll
-          for (int j = 0; j < DPL; ++j) acc[r][j] *= al;
-        }
-      }
-      const int n_tok = min(kGenTile, t_end - t0);
-      for (int tt = grp; tt < n_tok; tt += G) {
-        const T* vrow = vp + (size_t)(t0 + tt) * D;
-        float vv[DPL];
-#pragma unroll
-        for (int j = 0; j < DPL; ++j) vv[j] = E::ld(vrow + col + j * DL);
-#pragma unroll
-        for (int r = 0; r < kMaxRep; ++r) {
-          if (r >= n_rep) continue;
-          const float pr = p_s[r][tt];
-#pragma unroll
-          for (int j = 0; j < DPL; ++j) acc[r][j] += pr * vv[j];
-        }
-      }
-    }
-    // Block mass (accumulate mode): lane r sums its head's weights token by token, in order,
-    // and writes sum / l at the last token of each block (or of the wave's range).
-    if constexpr (kMass) {
-      if (lane < n_rep) {
-        const int r = lane;
-        const int n_tok = min(kGenTile, t_end - t0);
-        float bs = 0.f;
-#pragma unroll
-        for (int q = 0; q < kMaxRep; ++q)
-          if (q == r) bs = blk[q];
-        const int qh = h * n_rep + r;
-        for (int tt = 0; tt < n_tok; ++tt) {
-          bs += praw_s[r][tt];
-          const int tok = t0 + tt;
-          if ((tok + 1) % a.tokens_per_block == 0 || tok + 1 == t_end) {
-            a.block_mass[((size_t)b * a.hq + qh) * a.max_blocks + a.block_id_offset + tok / a.tokens_per_block] =
-                bs / l_run_at(l_run, r);
-            bs = 0.f;
-          }
-        }
-#pragma unroll
-        for (int q = 0; q < kMaxRep; ++q)
-          if (q == r) blk[q] = bs;
-      }
-    }
-    __syncthreads();
-  }
-
-  // Partials: token groups summed across lanes (xor over the group bits of the lane id).
-  const size_t slot = ((size_t)b * a.hkv + h) * a.n_split + split;
-#pragma unroll
-  for (int r = 0; r < kMaxRep; ++r) {
-    if (r >= n_rep) continue;
-    if constexpr (kWithV) {
-#pragma unroll
-      for (int j = 0; j < DPL; ++j) {
-        float x = acc[r][j];
-#pragma unroll
-        for (int o = DL; o < 64; o <<= 1) x += __shfl_xor(x, o);
-        if (grp == 0) a.pacc[(slot * n_rep + r) * D + col + j * DL] = x;
-      }
-    }
-    if constexpr (kFold) {
-      if (lane == 0) {
-        a.pm[slot * n_rep + r] = m_run[r];
-        a.pl[slot * n_rep + r] = l_run[r];
-      }
-    }
-  }
+  wg_merge_store<D, kFold, kWithV, false, DR>(sm, wave, g, n, m_run, l_run, acc, a.n_rep, a.pm + slot * a.n_rep,
+                                              a.pl + slot * a.n_rep, a.pacc + slot * a.n_rep * DR);
 }
 
 // Combine the dense partials into the caller's running state, in place.
@@ -1492,21 +1376,21 @@ hipError_t launch_dense_merge(const DenseArgs& a, int mode, int batch, int d, fl
   return hipGetLastError();
 }
 
-template <class Ty, int D>
+template <class Ty, int D, int DR>
 hipError_t launch_dense_t(const DenseArgs& a, int mode, int batch, hipStream_t stream) {
   dim3 grid(a.n_split, a.hkv, batch);
   switch (mode) {
     case kModeFold:
-      dense_attn_kernel<Ty, D, kModeFold><<<grid, 256, 0, stream>>>(a);
+      dense_attn_kernel<Ty, D, DR, kModeFold><<<grid, 256, 0, stream>>>(a);
       break;
     case kModeStats:
-      dense_attn_kernel<Ty, D, kModeStats><<<grid, 256, 0, stream>>>(a);
+      dense_attn_kernel<Ty, D, DR, kModeStats><<<grid, 256, 0, stream>>>(a);
       break;
     case kModeAccumulate:
-      dense_attn_kernel<Ty, D, kModeAccumulate><<<grid, 256, 0, stream>>>(a);
+      dense_attn_kernel<Ty, D, DR, kModeAccumulate><<<grid, 256, 0, stream>>>(a);
       break;
     default:
-      dense_attn_kernel<Ty, D, kModeFoldFixed><<<grid, 256, 0, stream>>>(a);
+      dense_attn_kernel<Ty, D, DR, kModeFoldFixed><<<grid, 256, 0, stream>>>(a);
       break;
   }
   return hipGetLastError();
@@ -1515,62 +1399,18 @@ hipError_t launch_dense_t(const DenseArgs& a, int mode, int batch, hipStream_t s
 template <class Ty>
 hipError_t launch_dense_ty(const DenseArgs& a, int mode, int batch, int d, hipStream_t stream) {
   switch (d) {
-    case 32:
-      return launch_dense_t<Ty, 32>(a, mode, batch, stream);
-    case 64:
-      return launch_dense_t<Ty, 64>(a, mode, batch, stream);
-    default:
-      return launch_dense_t<Ty, 128>(a, mode, batch, stream);
-  }
-}
-
-template <class E, int D>
-hipError_t launch_generic_t(const DenseArgs& a, int mode, int batch, hipStream_t stream) {
-  dim3 grid(a.n_split, a.hkv, batch);
-  switch (mode) {
-    case kModeFold:
-      dense_generic_kernel<E, D, kModeFold><<<grid, 64, 0, stream>>>(a);
-      break;
-    case kModeStats:
-      dense_generic_kernel<E, D, kModeStats><<<grid, 64, 0, stream>>>(a);
-      break;
-    case kModeAccumulate:
-      dense_generic_kernel<E, D, kModeAccumulate><<<grid, 64, 0, stream>>>(a);
-      break;
-    default:
-      dense_generic_kernel<E, D, kModeFoldFixed><<<grid, 64, 0, stream>>>(a);
-      break;
-  }
-  return hipGetLastError();
-}
-
-// 16-bit q/k/v at the head dims the MFMA kernel does not take.
-template <class Ty>
-hipError_t launch_generic_16(const DenseArgs& a, int mode, int batch, int d, hipStream_t stream) {
-  switch (d) {
     case 8:
-      return launch_generic_t<GenElem<Ty>, 8>(a, mode, batch, stream);
+      return launch_dense_t<Ty, 16, 8>(a, mode, batch, stream);
     case 16:
-      return launch_generic_t<GenElem<Ty>, 16>(a, mode, batch, stream);
-    default:
-      return launch_generic_t<GenElem<Ty>, 256>(a, mode, batch, stream);
-  }
-}
-
-hipError_t launch_generic_32(const DenseArgs& a, int mode, int batch, int d, hipStream_t stream) {
-  switch (d) {
-    case 8:
-      return launch_generic_t<F32Elem, 8>(a, mode, batch, stream);
-    case 16:
-      return launch_generic_t<F32Elem, 16>(a, mode, batch, stream);
+      return launch_dense_t<Ty, 16, 16>(a, mode, batch, stream);
     case 32:
-      return launch_generic_t<F32Elem, 32>(a, mode, batch, stream);
+      return launch_dense_t<Ty, 32, 32>(a, mode, batch, stream);
     case 64:
-      return launch_generic_t<F32Elem, 64>(a, mode, batch, stream);
+      return launch_dense_t<Ty, 64, 64>(a, mode, batch, stream);
     case 128:
-      return launch_generic_t<F32Elem, 128>(a, mode, batch, stream);
+      return launch_dense_t<Ty, 128, 128>(a, mode, batch, stream);
     default:
-      return launch_generic_t<F32Elem, 256>(a, mode, batch, stream);
+      return launch_dense_t<Ty, 256, 256>(a, mode, batch, stream);
   }
 }
 
@@ -1623,28 +1463,18 @@ void launch_merge_d(const PagedArgs& a, int stride, int d, dim3 grid, hipStream_
 
 }  // namespace
 
-bool head_dim_supported(int d) { return d == 32 || d == 64 || d == 128; }
+bool paged_head_dim_supported(int d) { return d == 16 || d == 32 || d == 64 || d == 128 || d == 256; }
 
-bool paged_head_dim_supported(int d) { return d == 16 || head_dim_supported(d) || d == 256; }
+bool dense_head_dim_supported(int d) { return d == 8 || paged_head_dim_supported(d); }
 
-bool dense_head_dim_supported(int d) { return d == 8 || d == 16 || head_dim_supported(d) || d == 256; }
-
-bool dense_generic(int dtype, int d) { return dtype == kF32 || !head_dim_supported(d); }
-
-int dense_waves_per_workgroup(int dtype, int d) { return dense_generic(dtype, d) ? 1 : kWaves; }
-
-int dense_wave_tokens(int dtype, int d, int batch, int hkv, int tc, int tokens_per_block, bool mass) {
-  // Aim for about 2048 waves over the grid (8 per CU; 1024 one-wave workgroups for the
-  // generic kernel), each folding at least one tile (16 tokens in the MFMA kernel, 64 in the
-  // generic one).
-  const bool gen = dense_generic(dtype, d);
-  const long tile = gen ? kGenTile : 16;
-  const long target = gen ? 1024 : 2048;
-  const long tiles = (tc + tile - 1) / tile;
+int dense_wave_tokens(int batch, int hkv, int tc, int tokens_per_block, bool mass) {
+  // Aim for about 2048 waves over the grid (8 per CU), each folding at least one 16-token tile.
+  const long target = 2048;
+  const long tiles = (tc + 15) / 16;
   const long rows = (long)batch * hkv;
   long per_wave = (tiles * rows + target - 1) / target;
   if (per_wave < 1) per_wave = 1;
-  long tokens = per_wave * tile;
+  long tokens = per_wave * 16;
   if (mass) {
     const long tpb = tokens_per_block;
     tokens = (tokens + tpb - 1) / tpb * tpb;
@@ -1654,9 +1484,9 @@ int dense_wave_tokens(int dtype, int d, int batch, int hkv, int tc, int tokens_p
 
 hipError_t launch_dense(int dtype, int mode, int d, const DenseLaunch& p, hipStream_t stream) {
   DenseArgs a;
-  a.q = static_cast<const uint16_t*>(p.q);
-  a.k = static_cast<const uint16_t*>(p.k);
-  a.v = static_cast<const uint16_t*>(p.v);
+  a.q = static_cast<const char*>(p.q);
+  a.k = static_cast<const char*>(p.k);
+  a.v = static_cast<const char*>(p.v);
   a.valid = p.valid;
   a.active = p.active;
   a.m_in = p.m;
@@ -1678,14 +1508,12 @@ hipError_t launch_dense(int dtype, int mode, int d, const DenseLaunch& p, hipStr
   a.softcap = p.softcap;
   hipError_t e;
   if (p.ev_start != nullptr && (e = hipEventRecord(p.ev_start, stream)) != hipSuccess) return e;
-  if (dtype == kF32)
-    e = launch_generic_32(a, mode, p.batch, d, stream);
-  else if (!head_dim_supported(d))
-    e = dtype == kF16 ? launch_generic_16<F16>(a, mode, p.batch, d, stream)
-                      : launch_generic_16<BF16>(a, mode, p.batch, d, stream);
+  if (dtype == kF16)
+    e = launch_dense_ty<F16>(a, mode, p.batch, d, stream);
+  else if (dtype == kBF16)
+    e = launch_dense_ty<BF16>(a, mode, p.batch, d, stream);
   else
-    e = dtype == kF16 ? launch_dense_ty<F16>(a, mode, p.batch, d, stream)
-                      : launch_dense_ty<BF16>(a, mode, p.batch, d, stream);
+    e = launch_dense_ty<F32>(a, mode, p.batch, d, stream);
   if (e != hipSuccess) return e;
   if (p.ev_stop != nullptr && (e = hipEventRecord(p.ev_stop, stream)) != hipSuccess) return e;
   if (p.attention_only) return hipSuccess;

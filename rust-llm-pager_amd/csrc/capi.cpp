@@ -58,14 +58,12 @@ struct DensePlan {
   size_t bytes = 0, o_pm = 0, o_pl = 0, o_pacc = 0;
 };
 
-DensePlan plan_dense(int64_t batch, int64_t hq, int64_t hkv, int64_t tokens, int64_t d, int mode, int64_t tpb,
-                     int dtype) {
+DensePlan plan_dense(int64_t batch, int64_t hq, int64_t hkv, int64_t tokens, int64_t d, int mode, int64_t tpb) {
   DensePlan p;
   if (tokens <= 0 || batch <= 0) return p;
   const bool mass = mode == PGR_MODE_ACCUMULATE;
-  p.wave_tokens =
-      pgr::dense_wave_tokens(dtype, (int)d, (int)batch, (int)hkv, (int)tokens, (int)(mass ? tpb : 16), mass);
-  const int64_t per_wg = (int64_t)pgr::dense_waves_per_workgroup(dtype, (int)d) * p.wave_tokens;
+  p.wave_tokens = pgr::dense_wave_tokens((int)batch, (int)hkv, (int)tokens, (int)(mass ? tpb : 16), mass);
+  const int64_t per_wg = (int64_t)pgr::kWaves * p.wave_tokens;
   p.n_split = (int)((tokens + per_wg - 1) / per_wg);
   const size_t slots = (size_t)batch * hkv * p.n_split;
   const size_t n_rep = (size_t)(hq / hkv);
@@ -149,7 +147,7 @@ int run_dense(int mode, const void* q, const void* k, const void* v, const int32
   if (tokens == 0 || batch == 0) return pgr::kOk;  // nothing to fold: the state is unchanged
   if (!q || !k || !m || !l || (mode != PGR_MODE_STATS && (!v || !acc)))
     return set_err(pgr::kErrInvalid, "null tensor pointer");
-  const DensePlan p = plan_dense(batch, hq, hkv, tokens, d, mode, tpb, dtype);
+  const DensePlan p = plan_dense(batch, hq, hkv, tokens, d, mode, tpb);
   if (ws == nullptr || ws_bytes < p.bytes) return set_err(pgr::kErrCapacity, "workspace too small");
   pgr::DenseLaunch L = dense_launch(p, q, k, v, valid, active, m, l, acc, block_mass, max_blocks, block_id_offset, tpb,
                                     batch, hq, hkv, tokens, scale, softcap, ws);
@@ -255,13 +253,7 @@ size_t pgr_attn_workspace_bytes(int64_t batch, int64_t num_query_heads, int64_t 
   try {
     if (batch <= 0 || num_kv_heads <= 0 || num_query_heads <= 0 || tokens <= 0 || head_dim <= 0) return 0;
     if (mode == PGR_MODE_ACCUMULATE && (tokens_per_block <= 0 || tokens_per_block % 16 != 0)) return 0;
-    // The geometry depends on the element type only at head dims 32/64/128 (16-bit there runs the
-    // MFMA kernel, fp32 the generic one): the size covers both.
-    const size_t a = plan_dense(batch, num_query_heads, num_kv_heads, tokens, head_dim, mode, tokens_per_block,
-                                pgr::kF16).bytes;
-    const size_t b = plan_dense(batch, num_query_heads, num_kv_heads, tokens, head_dim, mode, tokens_per_block,
-                                pgr::kF32).bytes;
-    return a > b ? a : b;
+    return plan_dense(batch, num_query_heads, num_kv_heads, tokens, head_dim, mode, tokens_per_block).bytes;
   } catch (...) {
     exception_status();
     return 0;
@@ -292,7 +284,7 @@ int pgr_attn_bench_step(const void* q, const void* const* k, const void* const* 
       return set_err(pgr::kErrInvalid, "pgr_attn_bench_step: inputs, chunks > 0, reps > 0 and outputs required");
     for (int c = 0; c < n_chunks; ++c)
       if (!k[c] || !v[c]) return set_err(pgr::kErrInvalid, "pgr_attn_bench_step: a null chunk");
-    const DensePlan p = plan_dense(batch, num_query_heads, num_kv_heads, tokens, head_dim, PGR_MODE_FOLD, 16, dtype);
+    const DensePlan p = plan_dense(batch, num_query_heads, num_kv_heads, tokens, head_dim, PGR_MODE_FOLD, 16);
     if (workspace == nullptr || workspace_bytes < p.bytes) return set_err(pgr::kErrCapacity, "workspace too small");
     hipEvent_t ev[2] = {nullptr, nullptr};
     hipError_t e = hipSuccess;
@@ -334,7 +326,7 @@ int pgr_attn_step_noalloc(const void* q, const void* k, const void* v, const int
     // with active = 0 is skipped by both), so nothing left in `scratch` by an earlier call is
     // read and nothing needs clearing.
     const size_t need =
-        plan_dense(batch, num_query_heads, num_kv_heads, tokens, head_dim, PGR_MODE_FOLD, 16, dtype).bytes;
+        plan_dense(batch, num_query_heads, num_kv_heads, tokens, head_dim, PGR_MODE_FOLD, 16).bytes;
     if (need > kNoAllocScratchBytes)
       return set_err(pgr::kErrCapacity, "pgr_attn_step_noalloc: this chunk needs " + std::to_string(need) +
                                             " bytes of split-K partials, more than the " +

@@ -17,10 +17,10 @@ Conventions kept from the reference:
 Differences, by design: p is rounded to the K/V dtype before P.V exactly as the reference
 does, but the chunk is folded by many workgroups in parallel and merged, so fp32 results
 differ from the reference's sequential fold in the last bits. q/k/v may be float16, bfloat16
-or float32, and head_dim one of 8, 16, 32, 64, 128, 256 (NotImplementedError otherwise);
-16-bit inputs at head_dim 32/64/128 run the MFMA kernel, the rest a VALU kernel. The
-reference zero-pads Q and K to 16 columns below head_dim 16 so that tl.dot applies
-(:56-66, :125-133); the dot products are the same without the padding. A masked position
+or float32, and head_dim one of 8, 16, 32, 64, 128, 256 (NotImplementedError otherwise), all
+on the matrix cores (fp32 with fp32 products and P unrounded). The reference zero-pads Q and K
+to 16 columns below head_dim 16 so that tl.dot applies (:56-66, :125-133); the kernel pads the
+same columns in registers. A masked position
 contributes exactly zero in every kernel, also when the fixed max m is -inf.
 """
 from __future__ import annotations
