@@ -72,10 +72,10 @@ int pgr_attn_step(const void* q, const void* k, const void* v, const int32_t* va
  * device array of the library (8 MiB per GPU, held until the process ends) instead of a
  * workspace. It calls no allocating routine. A chunk whose partials exceed 8 MiB is
  * rejected with PGR_ERR_CAPACITY. With fp16/bf16 q/k/v, chunks with batch * num_kv_heads
- * <= 496 always fit at head_dim <= 128 and n_rep <= 16. fp32 q/k/v run a kernel with more,
- * smaller partial slots: there chunks with batch * num_kv_heads <= 496 always fit while
+ * <= 496 always fit at head_dim <= 128 and n_rep <= 16. fp32 q/k/v count as more, smaller
+ * partial slots: there chunks with batch * num_kv_heads <= 496 always fit while
  * head_dim * n_rep <= 1024 (head_dim 64 at n_rep 16, 128 at n_rep 8); at head_dim 128 with
- * n_rep 16 a long chunk of even one row is rejected (1 x 16 x 65536 x 128 needs 8.5 MB).
+ * n_rep 16 a long chunk of even one row is rejected (1 x 16 x 65536 x 128 counts as 8.5 MB).
  * Calls share their GPU's array. Outside graph capture the library orders them: a call on
  * another stream than the previous call's waits on the GPU (hipStreamWaitEvent) for the
  * previous call to finish, so calls from several streams or threads run one after another

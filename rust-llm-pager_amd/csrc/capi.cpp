@@ -78,6 +78,22 @@ DensePlan plan_dense(int64_t batch, int64_t hq, int64_t hkv, int64_t tokens, int
   return p;
 }
 
+// The size of a chunk that pgr_attn_step_noalloc accepts is part of its contract (pgr.h) and
+// does not follow the kernels' plans: bytes of split-K partials at 16 tokens per wave and up,
+// four waves per slot, about 2048 waves (16-bit q/k/v at head dims 32, 64 and 128), or at 64
+// tokens per slot and up, about 1024 slots (fp32 and the other head dims). Never less than
+// plan_dense needs.
+size_t noalloc_contract_bytes(int64_t batch, int64_t hq, int64_t hkv, int64_t tokens, int64_t d, int dtype) {
+  const bool mid = dtype != pgr::kF32 && (d == 32 || d == 64 || d == 128);
+  const int64_t rows = batch * hkv, tile = mid ? 16 : 64, waves = mid ? 4 : 1, target = mid ? 2048 : 1024;
+  const int64_t tiles = (tokens + tile - 1) / tile;
+  const int64_t per_slot = waves * tile * ((tiles * rows + target - 1) / target);
+  const size_t slots = (size_t)rows * (size_t)((tokens + per_slot - 1) / per_slot);
+  const size_t n_rep = (size_t)(hq / hkv);
+  return 2 * pgr::align_up(slots * n_rep * sizeof(float), 256) +
+         pgr::align_up(slots * n_rep * (size_t)d * sizeof(float), 256);
+}
+
 // Launch timing of the operator API's attention kernel (pgr_attn_set_timing): fence-free
 // events around each fold launch, resolved by pgr_attn_kernel_time. One process-wide list.
 struct DenseTiming {
@@ -325,8 +341,7 @@ int pgr_attn_step_noalloc(const void* q, const void* k, const void* v, const int
     // Every partial slot that the merge reads is written by the fold launch before it (a row
     // with active = 0 is skipped by both), so nothing left in `scratch` by an earlier call is
     // read and nothing needs clearing.
-    const size_t need =
-        plan_dense(batch, num_query_heads, num_kv_heads, tokens, head_dim, PGR_MODE_FOLD, 16).bytes;
+    const size_t need = noalloc_contract_bytes(batch, num_query_heads, num_kv_heads, tokens, head_dim, dtype);
     if (need > kNoAllocScratchBytes)
       return set_err(pgr::kErrCapacity, "pgr_attn_step_noalloc: this chunk needs " + std::to_string(need) +
                                             " bytes of split-K partials, more than the " +
