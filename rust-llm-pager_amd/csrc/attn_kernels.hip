@@ -1064,18 +1064,24 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const WorkItem* __restr
 // output and the final (m, l) for the mass pass are written. The kernel is latency-bound:
 // each thread issues a whole batch of partial loads before using any of them (a load past
 // the last partial re-reads it and is weighted 0).
+//
+// kU, slots per thread and batch: the smallest of 1, 2, 4, 8, 16 whose one batch covers every
+// slot range of the step (16, in several batches, beyond that and for packed slots). Slots past
+// a sequence's count add exact zeros, so the sums do not depend on it; fewer of them are loads
+// and exponentials the kernel does without. Per layer (attention and merge), 64 sequences of 93
+// to 2038 tokens at head dim 128 (14 slots at most): 25.6 us with 16 slots per thread, 23.3 with
+// 4; with block mass 27.2 and 24.7. 8 sequences at head dim 64 (74 slots): 16 per thread still.
 constexpr int kMergeBatch = 16;
 
 // The leading arguments are preloaded into SGPRs (as in paged_attn_kernel): the partial loads
 // of the first batch depend on nothing else, and go out before the plan's SeqInfo arrives.
-template <class Ty, int D>
+template <class Ty, int D, int kU>
 __global__ __launch_bounds__(256) void paged_merge_kernel(const SeqInfo* __restrict__ seqs, const float* pm0,
                                                           const float* pl0, const float* pacc0,
                                                           int partial_stride, int hq, int n_rep, int hkv,
                                                           PagedArgs a) {
   constexpr int kLanes = D / 2;          // threads per partial group (two dims each)
   constexpr int G = 256 / kLanes;        // partial groups
-  constexpr int kU = kMergeBatch;
   constexpr int kRed = kLanes < kWaveSize ? kLanes : kWaveSize;  // lanes of group 0 per wave
   __shared__ float m_s[G], l_s[G];
   __shared__ float acc_s[G][D];
@@ -1120,6 +1126,14 @@ __global__ __launch_bounds__(256) void paged_merge_kernel(const SeqInfo* __restr
   }
 
   const int P = si->partial_count;  // P >= 1: every sequence has a work item
+  // Deferred mass: the thread's first block's entries, loaded beside the partials.
+  const size_t mass_row = ((size_t)seq * hq + qh) * a.mass_stride;
+  const int mass_b0 = si->mass_lo + tid, n_mass = a.mass_w != nullptr ? si->n_mass : 0;
+  float mass_m0 = 0.f, mass_s0 = 0.f;
+  if (mass_b0 < n_mass) {
+    mass_m0 = a.mass_m[mass_row + mass_b0];
+    mass_s0 = a.mass_s[mass_row + mass_b0];
+  }
   const int h = qh / n_rep;
   const size_t kv_row = ((size_t)seq * hkv + h) * D;
   if (seq == 0 && qh == 0 && tid == 0) {
@@ -1232,12 +1246,9 @@ __global__ __launch_bounds__(256) void paged_merge_kernel(const SeqInfo* __restr
   // all threads. Blocks below mass_lo keep the 0 the last step's reduction left.
   __syncthreads();
   const float mfin = fin_s[0], lfin = fin_s[1];
-  const size_t row = (size_t)seq * hq + qh;
-  const int n_mass = si->n_mass;
-  for (int b = si->mass_lo + tid; b < n_mass; b += 256) {
-    const size_t mi = row * a.mass_stride + b;
-    a.mass_w[mi] = a.mass_s[mi] * __builtin_amdgcn_exp2f(a.mass_m[mi] - mfin) / lfin;
-  }
+  if (mass_b0 < n_mass) a.mass_w[mass_row + mass_b0] = mass_s0 * __builtin_amdgcn_exp2f(mass_m0 - mfin) / lfin;
+  for (int b = mass_b0 + 256; b < n_mass; b += 256)
+    a.mass_w[mass_row + b] = a.mass_s[mass_row + b] * __builtin_amdgcn_exp2f(a.mass_m[mass_row + b] - mfin) / lfin;
 }
 
 // Per (session, block): mean over the session's rows and all query heads of
@@ -1441,23 +1452,40 @@ hipError_t launch_paged_d(const PagedArgs& a, int d, int n_work, bool mass, hipS
   }
 }
 
+template <class Ty, int D>
+void launch_merge_t(const PagedArgs& a, int stride, dim3 grid, hipStream_t stream) {
+  constexpr int G = 512 / D;  // thread groups of the kernel
+  const int per_group = stride > 0 ? (stride + G - 1) / G : kMergeBatch;
+  if (per_group <= 1)
+    paged_merge_kernel<Ty, D, 1><<<grid, 256, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep, a.hkv, a);
+  else if (per_group <= 2)
+    paged_merge_kernel<Ty, D, 2><<<grid, 256, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep, a.hkv, a);
+  else if (per_group <= 4)
+    paged_merge_kernel<Ty, D, 4><<<grid, 256, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep, a.hkv, a);
+  else if (per_group <= 8)
+    paged_merge_kernel<Ty, D, 8><<<grid, 256, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep, a.hkv, a);
+  else
+    paged_merge_kernel<Ty, D, kMergeBatch><<<grid, 256, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep,
+                                                                     a.hkv, a);
+}
+
 template <class Ty>
 void launch_merge_d(const PagedArgs& a, int stride, int d, dim3 grid, hipStream_t stream) {
   switch (d) {
     case 16:
-      paged_merge_kernel<Ty, 16><<<grid, 256, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep, a.hkv, a);
+      launch_merge_t<Ty, 16>(a, stride, grid, stream);
       break;
     case 32:
-      paged_merge_kernel<Ty, 32><<<grid, 256, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep, a.hkv, a);
+      launch_merge_t<Ty, 32>(a, stride, grid, stream);
       break;
     case 64:
-      paged_merge_kernel<Ty, 64><<<grid, 256, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep, a.hkv, a);
+      launch_merge_t<Ty, 64>(a, stride, grid, stream);
       break;
     case 128:
-      paged_merge_kernel<Ty, 128><<<grid, 256, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep, a.hkv, a);
+      launch_merge_t<Ty, 128>(a, stride, grid, stream);
       break;
     default:
-      paged_merge_kernel<Ty, 256><<<grid, 256, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep, a.hkv, a);
+      launch_merge_t<Ty, 256>(a, stride, grid, stream);
   }
 }
 
