@@ -76,13 +76,38 @@ struct BF16 {
   static __device__ __forceinline__ float to_f(uint16_t x) { return __builtin_bit_cast(float, (uint32_t)x << 16); }
 };
 
+// Max / sum over the four lane groups g (rows of 16 lanes), in every lane. v_permlane16_swap
+// exchanges the odd rows of its first operand with the even rows of its second, and
+// v_permlane32_swap the halves: with x in both, the two results hold x of the two rows (halves)
+// of each pair. Two VALU moves where __shfl_xor is an LDS permute and a wait on the tile's
+// dependence chain; the same pairs are added in the same order.
+// (The result's elements are read into scalars first: __builtin_bit_cast of a vector element
+// takes element 0.)
+__device__ __forceinline__ void row_pair(float x, float& a, float& b) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const uint32_t r0 = r[0], r1 = r[1];
+  a = __builtin_bit_cast(float, r0);
+  b = __builtin_bit_cast(float, r1);
+}
+__device__ __forceinline__ void half_pair(float x, float& a, float& b) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const uint32_t r0 = r[0], r1 = r[1];
+  a = __builtin_bit_cast(float, r0);
+  b = __builtin_bit_cast(float, r1);
+}
 __device__ __forceinline__ float wave_max_g(float x) {
-  x = fmaxf(x, __shfl_xor(x, 16));
-  return fmaxf(x, __shfl_xor(x, 32));
+  float a, b;
+  row_pair(x, a, b);
+  half_pair(fmaxf(a, b), a, b);
+  return fmaxf(a, b);
 }
 __device__ __forceinline__ float wave_sum_g(float x) {
-  x += __shfl_xor(x, 16);
-  return x + __shfl_xor(x, 32);
+  float a, b;
+  row_pair(x, a, b);
+  half_pair(a + b, a, b);
+  return a + b;
 }
 
 // fp32 q/k/v (the dense operator kernels only): one dword per operand and lane.
@@ -781,9 +806,16 @@ __device__ __forceinline__ void pv_tile_t(f32x4 (&acc)[D / 16], const PTile<D>& 
 }
 
 struct TileMeta {
-  int t0;        // first token position of the tile
-  int block_id;
-  int last;      // last tile of its block
+  int t0;    // first token position of the tile
+  int unit;  // kMass: the mass unit that ends with this tile, or -1
+};
+
+// Mass launches: units a work item's blocks hold at most (tiles, or whole blocks where that
+// would be more). (m, s) of 128 units take 16 KB of LDS; 64 at head dim 256, whose workgroup
+// merge takes 66 KB, so that two workgroups fit a CU.
+template <int D>
+struct MassUnits {
+  static constexpr int N = D == 256 ? 2 * kMaxWorkEntries : 4 * kMaxWorkEntries;
 };
 
 // Mirror mode: most reads of a layer's "mirror filled" word before a workgroup reads the host
@@ -804,9 +836,9 @@ template <class Ty, int D, bool kMass>
 __global__ __launch_bounds__(256) void paged_attn_kernel(const WorkItem* __restrict__ work, uint16_t* pool,
                                                          const uint16_t* stage, PagedArgs a) {
   constexpr int NB = PagedRing<D>::NB;
-  constexpr int kWaveEntries = kMaxWorkEntries / kWaves;  // entries one wave folds at most
+  constexpr int kUnits = kMass ? MassUnits<D>::N : 1;
   __shared__ MergeSmem<D> sm;
-  __shared__ float mass_sm[kMass ? kWaves : 1][kWaveEntries][2][kMaxRep];
+  __shared__ float mass_m_sm[kUnits][kMaxRep], mass_s_sm[kUnits][kMaxRep];
   const WorkItem* wi = work + blockIdx.x;
   const int h = blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -843,29 +875,34 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const WorkItem* __restr
       static_cast<u32x4*>(a.aux_dst)[v] = static_cast<const u32x4*>(a.aux_src)[v];
   }
 
-  // The work item's blocks hold count * tpb tiles, flat index x = entry * tpb + tile in
-  // block. With per-block mass (kMass) wave w folds whole blocks: entries w, w+4, w+8, ...
-  // (a block's mass is then one wave's). Otherwise it folds tiles x = w, w+4, w+8, ..., so
-  // that the four waves' tile counts differ by at most one and no wave holds the workgroup
-  // up by a whole block. The cursor (fe, ftb) names the next fetch's entry and tile in
+  // The work item's blocks hold count * tpb tiles, flat index x = entry * tpb + tile in block.
+  // Wave w folds tiles x = w, w+4, w+8, ..., so that the four waves' tile counts differ by at
+  // most one and no wave holds the workgroup up by a whole block. With per-block mass (kMass)
+  // a tile's (m, s) is one unit in LDS, and a block's units are combined after the loop; where
+  // the blocks hold too many tiles for that, wave w folds whole blocks: entries w, w+4, ...
+  // (a unit is then a block). Against whole blocks dealt to the waves at every block size:
+  // 64 sequences at head dim 128 (32-token blocks) 23.15 -> 22.87 us per layer, 8 sequences up to
+  // 28770 tokens at head dim 64 23.0 -> 22.5, 4 of 32768 at head dim 128 99.9 -> 99.6. The cursor (fe, ftb) names the next fetch's entry and tile in
   // block; the entry being fetched and the next one sit in SGPRs, and the one after is read
-  // (a scalar load) as a fetch is issued, a fetch or a block ahead of its use. Entries past
-  // entry_count are never read by a fetch (the slots exist in every work item).
-  int fe = kMass ? 0 : wave / tpb, ftb = kMass ? 0 : wave - (wave / tpb) * tpb;
-  const int step_e = kWaves / tpb, step_tb = kWaves - step_e * tpb;  // x += kWaves (no kMass)
+  // (a scalar load) as a fetch is issued, a fetch ahead of its use. Entries past entry_count
+  // are never read by a fetch (the slots exist in every work item).
+  const bool by_tile = !kMass || tpb * kMaxWorkEntries <= kUnits;
+  int fe = by_tile ? wave / tpb : wave, ftb = by_tile ? wave - (wave / tpb) * tpb : 0;
+  const int step_e = by_tile ? kWaves / tpb : 0, step_tb = by_tile ? kWaves - step_e * tpb : 1;
+  const int wrap_e = by_tile ? 1 : kWaves;
   auto advance = [&](int& e, int& tb) {
     tb += step_tb;
     e += step_e;
     if (tb >= tpb) {
       tb -= tpb;
-      ++e;
+      e += wrap_e;
     }
   };
   auto entry_at = [&](int e) { return wi->entries[e < kMaxWorkEntries ? e : kMaxWorkEntries - 1]; };
   int ne = fe, ntb = ftb;  // the fetch after the next one
-  if (!kMass) advance(ne, ntb);
-  BlockEntry ecur = kMass ? wi->entries[wave] : entry_at(fe);
-  BlockEntry enxt = kMass ? wi->entries[wave + kWaves] : entry_at(ne);
+  advance(ne, ntb);
+  BlockEntry ecur = entry_at(fe);
+  BlockEntry enxt = entry_at(ne);
 
   // Mirror mode: host records come from the layer's HBM mirror, filled by DMA on the store's
   // copy stream, which sets the word after the layer's copies. One lane per workgroup polls
@@ -898,6 +935,7 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const WorkItem* __restr
   }
 
   RunVec<D> q[LaneRun<D>::N];  // loaded behind the first tile (below)
+  int mass_bid = 0;            // kMass: block of the entry this thread stores, behind q
 
   // Score transform: x = mult * s' with s' = s (no softcap) or cap * tanh(s * scale / cap).
   const bool capped = a.softcap > 0.f;
@@ -909,8 +947,9 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const WorkItem* __restr
 #pragma unroll
   for (int j = 0; j < D / 16; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int my_blocks = count > wave ? (count - wave + kWaves - 1) / kWaves : 0;
-  const int tiles = kMass ? my_blocks * tpb : (count * tpb > wave ? (count * tpb - wave + kWaves - 1) / kWaves : 0);
+  const int n_units = by_tile ? count * tpb : count;  // dealt to the waves in turn
+  const int my_units = n_units > wave ? (n_units - wave + kWaves - 1) / kWaves : 0;
+  const int tiles = by_tile ? my_units : my_units * tpb;
 
   // Next tile to fetch: the wave's nf-th. Every fetch in the loop is unconditional, so the
   // load counter stays in order; a fetch past the wave's last tile goes through an empty
@@ -930,23 +969,13 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const WorkItem* __restr
     const uint32_t sk = (uint32_t)(ftb * 16 * D * 2);
     load_tile_rs<D>(t, r, sk, sk + (uint32_t)(v_off * 2), k_lane, v_lane);
     mt.t0 = tt0;
-    mt.block_id = bid;
-    mt.last = (ftb == tpb - 1) ? fe : -1;
+    if constexpr (kMass) mt.unit = by_tile ? fe * tpb + ftb : (ftb == tpb - 1 ? fe : -1);
     ++nf;
-    if constexpr (kMass) {
-      if (++ftb == tpb) {
-        ftb = 0;
-        ++fe;
-        ecur = enxt;
-        if (fe + 1 < kWaveEntries) enxt = wi->entries[wave + (fe + 1) * kWaves];
-      }
-    } else {
-      fe = ne;
-      ftb = ntb;
-      ecur = enxt;
-      advance(ne, ntb);
-      enxt = entry_at(ne);
-    }
+    fe = ne;
+    ftb = ntb;
+    ecur = enxt;
+    advance(ne, ntb);
+    enxt = entry_at(ne);
   };
 
   auto fold = [&](PTile<D>& t, const TileMeta& mt) {
@@ -997,11 +1026,11 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const WorkItem* __restr
     pv_tile_t<Ty, D>(acc, t, p);
     if constexpr (kMass) {
       blk += psum;
-      if (mt.last >= 0) {  // block complete: (m_b, s_b) of this block to LDS, stored after the loop
-        const float bs = wave_sum_g(blk);
+      if (mt.unit >= 0) {  // unit complete: its (m, s) to LDS, combined and stored after the loop
+        const float us = wave_sum_g(blk);
         if (g == 0) {
-          mass_sm[wave][mt.last][0][n] = m_run;
-          mass_sm[wave][mt.last][1][n] = bs;
+          mass_m_sm[mt.unit][n] = m_run;
+          mass_s_sm[mt.unit][n] = us;
         }
         blk = 0.f;
       }
@@ -1016,6 +1045,7 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const WorkItem* __restr
     // the loop's wait counts independent of it while tiles 1 .. NB-2 stay in flight.
     fetch(buf[0], meta[0]);
     load_q_run<D>(q, a.q + ((size_t)seq * a.hq + qh) * D, real, g);
+    if constexpr (kMass) mass_bid = wi->entries[threadIdx.x % kMaxWorkEntries].block_id;
 #pragma unroll
     for (int j = 1; j < NB - 1; ++j) fetch(buf[j], meta[j]);
 #pragma unroll
@@ -1027,16 +1057,28 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const WorkItem* __restr
         if (ti + j < tiles) fold(buf[j], meta[j]);
       }
     }
+  } else if constexpr (kMass) {
+    mass_bid = wi->entries[threadIdx.x % kMaxWorkEntries].block_id;
   }
   if constexpr (kMass) {
-    if (g == 0 && real) {
-      for (int e = 0; e < my_blocks; ++e) {
-        const int bid = wi->entries[wave + e * kWaves].block_id;
-        if (bid < n_mass) {
-          const size_t mi = ((size_t)seq * a.hq + qh) * a.mass_stride + bid;
-          a.mass_m[mi] = mass_sm[wave][e][0][n];
-          a.mass_s[mi] = mass_sm[wave][e][1][n];
+    // Block mass: thread (e, r) combines the units of entry e for head r (under their largest
+    // max) and stores the block's (m, s). Consecutive threads take consecutive entries, whose
+    // blocks mostly follow each other in the head's row.
+    __syncthreads();
+    const int e = threadIdx.x % kMaxWorkEntries;
+    if (e < count && mass_bid < n_mass) {
+      const int per = by_tile ? tpb : 1;
+      for (int r = threadIdx.x / kMaxWorkEntries; r < a.n_rep; r += kWaves * kWaveSize / kMaxWorkEntries) {
+        float mb = mass_m_sm[e * per][r], sb = mass_s_sm[e * per][r];
+        for (int u = 1; u < per; ++u) {
+          const float mu = mass_m_sm[e * per + u][r], su = mass_s_sm[e * per + u][r];
+          const float mn = fmaxf(mb, mu);
+          sb = sb * __builtin_amdgcn_exp2f(mb - mn) + su * __builtin_amdgcn_exp2f(mu - mn);
+          mb = mn;
         }
+        const size_t mi = ((size_t)seq * a.hq + h * a.n_rep + r) * a.mass_stride + mass_bid;
+        a.mass_m[mi] = mb;
+        a.mass_s[mi] = sb;
       }
     }
   }
