@@ -1,4 +1,5 @@
-"""Build libpgr.so (HIP kernels + C++ host runtime + C ABI) in-tree for gfx950.
+"""Build libpgr.so (HIP kernels + C++ host runtime + C ABI) and _pgr_ops.so (the operator API's
+torch call path over it) in-tree for gfx950.
 
 Usage: python rust-llm-pager_amd/build.py [--jobs N] [--debug]
 """
@@ -14,6 +15,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libpgr.so")
+OPS_OUT = os.path.join(HERE, "_pgr_ops.so")
 OBJ_DIR = os.path.join(HERE, "_build")
 
 ARCH = "gfx950"
@@ -57,12 +59,35 @@ def compile_one(src: str, lang: str, extra: list[str], opt: list[str]) -> str:
     return obj
 
 
+def build_ops(opt: list[str]) -> None:
+    """The CPython module over torch's C++ API: host code only, g++ against the installed torch."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = OPS_OUT + ".tmp"
+    cmd = ["g++", "-shared", "-fPIC", "-std=c++17", *opt, "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    for path in [*include_paths(), sysconfig.get_paths()["include"]]:
+        cmd += ["-isystem", path]
+    cmd += [os.path.join(CSRC, "torch_ops.cpp"), "-o", tmp, "-L", lib, "-ltorch_python", "-ltorch_cpu", "-lc10",
+            f"-Wl,-rpath,{lib}"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, OPS_OUT)
+
+
 def build(jobs: int = 8, debug: bool = False) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     opt = ["-O1", "-g"] if debug else ["-O3"]
     with concurrent.futures.ThreadPoolExecutor(max_workers=max(1, jobs)) as pool:
         futures = [pool.submit(compile_one, s, lang, extra, opt) for s, lang, extra in SOURCES]
+        ops = pool.submit(build_ops, opt)
         objs = [f.result() for f in futures]
+        ops.result()
     tmp = OUT + ".tmp"
     cmd = [hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", tmp]
     res = subprocess.run(cmd, capture_output=True, text=True)

@@ -38,6 +38,26 @@ def stream_of(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def bind_ops():
+    """The _pgr_ops module (call path of the operator API for plain tensors), bound to the loaded
+    libpgr.so's entry points."""
+    import ctypes
+
+    try:
+        import _pgr_ops
+    except ImportError as e:
+        raise ImportError(f"_pgr_ops.so is missing or does not match this torch ({e}); build it with "
+                          "`python rust-llm-pager_amd/build.py` (or __graft_entry__.build())") from e
+    raw = _raw_stream
+    if raw is None:
+        def raw(index):
+            return torch.cuda.current_stream(index).cuda_stream
+    names = ("workspace_bytes", "step", "stats_step", "accumulate_step", "fold_fixed_step", "state_init", "finalize")
+    _pgr_ops.bind(*(ctypes.cast(getattr(lib(), "pgr_attn_" + n), ctypes.c_void_p).value for n in names), raw,
+                  torch.OutOfMemoryError)
+    return _pgr_ops
+
+
 def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 

@@ -29,6 +29,8 @@ import torch
 
 from . import _native as N
 
+_ops = N.bind_ops()  # plain tensors; None from any of its functions: the path below it decides
+
 _M_TILE = 16  # streaming_attention.py:55: query heads packed per KV head
 _QKV_CODES = {torch.float16: N.nat.DTYPE_F16, torch.bfloat16: N.nat.DTYPE_BF16, torch.float32: N.nat.DTYPE_F32}
 
@@ -104,6 +106,15 @@ def streaming_attention_state_init(batch_size: int, num_query_heads: int, head_d
     """Fresh online-softmax accumulator state, before any KV chunk has been folded in (:444-449):
     m = -inf, l = 0, acc = 0 in fp32, written by one native launch."""
     device = torch.device(device)
+    if device.type == "cuda":
+        if device.index is None:
+            device = torch.device("cuda", torch.cuda.current_device())
+        done = None
+        if torch.cuda.is_initialized():  # torch.empty below initializes it
+            done = _ops.state_init(batch_size, num_query_heads, head_dim, device)
+        if done is not None:
+            N.nat.check(done[0], "streaming_attention_state_init")
+            return done[1:]
     if device.type != "cuda":
         raise ValueError("streaming attention expects CUDA (HIP) tensors")
     m = torch.empty((batch_size, num_query_heads), dtype=torch.float32, device=device)
@@ -130,6 +141,10 @@ def streaming_attention_step(
     softcap: float | None = None,
 ) -> None:
     """Fold one KV chunk into the running (m, l, acc) state, in place (:452-513)."""
+    rc = _ops.step(q, k, v, m, l, acc, valid, active, scale, softcap)
+    if rc is not None:
+        N.nat.check(rc, "streaming_attention_step")
+        return
     b, hq, hkv, tc, d, code, dev, q, k, v, valid, active, scale = _prep(q, k, v, m, l, acc, valid, active, scale)
     if tc == 0 or b == 0:
         return
@@ -155,6 +170,10 @@ def streaming_attention_stats_step(
     softcap: float | None = None,
 ) -> None:
     """Pass 1: fold one KV chunk's K into running (m, l) only (:516-560)."""
+    rc = _ops.stats_step(q, k, m, l, valid, active, scale, softcap)
+    if rc is not None:
+        N.nat.check(rc, "streaming_attention_stats_step")
+        return
     b, hq, hkv, tc, d, code, dev, q, k, _, valid, active, scale = _prep(q, k, None, m, l, None, valid, active, scale)
     if tc == 0 or b == 0:
         return
@@ -184,6 +203,11 @@ def streaming_attention_accumulate_step(
     softcap: float | None = None,
 ) -> None:
     """Pass 2: fold one block-aligned KV group into acc and write its per-block mass (:563-621)."""
+    rc = _ops.accumulate_step(q, k, v, m, l, acc, block_mass, block_id_offset, tokens_per_block, valid, active, scale,
+                              softcap)
+    if rc is not None:
+        N.nat.check(rc, "streaming_attention_accumulate_step")
+        return
     b, hq, hkv, tc, d, code, dev, q, k, v, valid, active, scale = _prep(q, k, v, m, l, acc, valid, active, scale)
     _state(block_mass, "block_mass")
     N.require_cuda(block_mass)
@@ -215,6 +239,10 @@ def streaming_attention_fold_fixed_step(
     softcap: float | None = None,
 ) -> None:
     """Pass 2 fold for a non-block chunk (the tail): accumulate acc only, no mass (:624-665)."""
+    rc = _ops.fold_fixed_step(q, k, v, m, l, acc, valid, scale, softcap)
+    if rc is not None:
+        N.nat.check(rc, "streaming_attention_fold_fixed_step")
+        return
     b, hq, hkv, tc, d, code, dev, q, k, v, valid, _, scale = _prep(q, k, v, m, l, acc, valid, None, scale)
     if tc == 0 or b == 0:
         return
@@ -233,6 +261,10 @@ _FINALIZE_CODES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
 
 def streaming_attention_finalize(acc: torch.Tensor, l: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """(acc / l) cast to dtype, once every chunk has been folded in (:668-670)."""
+    done = _ops.finalize(acc, l, dtype)
+    if done is not None:
+        N.nat.check(done[0], "streaming_attention_finalize")
+        return done[1]
     if dtype not in _FINALIZE_CODES:
         raise NotImplementedError(f"finalize supports float16, bfloat16 and float32 outputs, got {dtype}")
     dev = N.require_cuda(acc, l)
