@@ -309,6 +309,84 @@ __device__ __forceinline__ void wg_merge_store(MergeSmem<D>& sm, int wave, int g
   }
 }
 
+// Workgroup merge of the four waves' (m, l, acc) straight into the caller's running state: the
+// workgroup holds the whole chunk of its heads (one split), so there are no partials to combine.
+// m_in: the state's m per head, read before any thread writes it. Fold: the state is one more
+// term of the online softmax; fixed: the sums are added to acc. Nothing valid in the chunk (and
+// none before) leaves the state as it was, as dense_merge_kernel does.
+template <int D, bool kFold, bool kWithAcc, int DR>
+__device__ __forceinline__ void wg_merge_state(MergeSmem<D>& sm, int wave, int g, int n, float m_run, float l_lane,
+                                               const f32x4 (&acc)[D / 16], int n_rep, const float* m_in, float* m,
+                                               float* l, float* state) {
+  constexpr int kThreads = kWaves * kWaveSize;
+  constexpr int kPer = kWithAcc ? (kMaxRep * DR + kThreads - 1) / kThreads : 1;  // state elements per thread
+  const int tid = threadIdx.x;
+  // The state's values load while the waves' sums go to LDS.
+  float old[kPer], l_old = 0.f;
+  if constexpr (kWithAcc) {
+#pragma unroll
+    for (int x = 0; x < kPer; ++x) {
+      const int idx = tid + x * kThreads;
+      old[x] = idx < n_rep * DR ? state[idx] : 0.f;
+    }
+  }
+  if (kFold && tid < n_rep) l_old = l[tid];
+  const float l_wave = wave_sum_g(l_lane);
+  if (g == 0) {
+    sm.m[wave][n] = m_run;
+    sm.l[wave][n] = l_wave;
+  }
+  if constexpr (kWithAcc) {
+#pragma unroll
+    for (int j = 0; j < D / 16; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sm.acc[wave][n][acc_dim<D>(g, i, j)] = acc[j][i];
+  }
+  __syncthreads();
+  auto final_max = [&](int r, float& m0) {
+    m0 = m_in[r];
+    float mf = m0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) mf = fmaxf(mf, sm.m[w][r]);
+    return mf;
+  };
+  if constexpr (kFold) {
+    if (tid < n_rep) {
+      float m0;
+      const float mf = final_max(tid, m0);
+      if (mf != kNegInf) {
+        float lf = l_old * __expf(m0 - mf);
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) lf += sm.l[w][tid] * __expf(sm.m[w][tid] - mf);
+        m[tid] = mf;
+        l[tid] = lf;
+      }
+    }
+  }
+  if constexpr (kWithAcc) {
+#pragma unroll
+    for (int x = 0; x < kPer; ++x) {
+      const int idx = tid + x * kThreads;
+      if (idx >= n_rep * DR) break;
+      const int r = idx / DR, d = idx - r * DR;
+      if constexpr (kFold) {
+        float m0;
+        const float mf = final_max(r, m0);
+        if (mf == kNegInf) continue;
+        float a = old[x] * __expf(m0 - mf);
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) a += sm.acc[w][r][d] * __expf(sm.m[w][r] - mf);
+        state[idx] = a;
+      } else {
+        float a = old[x];
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) a += sm.acc[w][r][d];
+        state[idx] = a;
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------------------
 // Dense chunk kernel: the operator API of pager_hf/streaming_attention.py:452-665.
 // k, v: [B, Hkv, Tc, D] contiguous. Grid (n_split, Hkv, B); each wave folds
@@ -330,6 +408,10 @@ struct DenseArgs {
   int tc, hq, hkv, n_rep, n_split, wave_tokens;
   int tokens_per_block, max_blocks, block_id_offset;
   float scale, softcap;
+  // One split: the caller's state, updated by the attention kernel itself (null: partials).
+  float* m_state;
+  float* l_state;
+  float* acc_state;
 };
 
 // Memory-bound at every type and head dim: K and V are read once, in 16-byte pieces where a
@@ -355,6 +437,7 @@ __global__ __launch_bounds__(256) void dense_attn_kernel(DenseArgs a) {
   constexpr bool kQLds = T::KD + 4 * T::VD > 64;
   constexpr int kQStride = D + 4;  // LDS q rows (kQLds): 16 bytes apart in banks
   __shared__ MergeSmem<D> sm;
+  __shared__ float m_old[kMaxRep];  // one split: the state's m before the chunk
 
   const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   if (a.active != nullptr && a.active[b] == 0) return;  // whole workgroup: uniform exit
@@ -522,45 +605,57 @@ __global__ __launch_bounds__(256) void dense_attn_kernel(DenseArgs a) {
     }
   }
 
+  if (a.m_state != nullptr) {  // read ahead of the workgroup merge's barrier
+    const size_t row = (size_t)b * a.hq + (size_t)h * a.n_rep;
+    if (kFold && threadIdx.x < (unsigned)a.n_rep) m_old[threadIdx.x] = a.m_state[row + threadIdx.x];
+    wg_merge_state<D, kFold, kWithV, DR>(sm, wave, g, n, m_run, l_run, acc, a.n_rep, m_old, a.m_state + row,
+                                         a.l_state + row, a.acc_state + row * DR);
+    return;
+  }
   const size_t slot = ((size_t)b * a.hkv + h) * a.n_split + split;
   wg_merge_store<D, kFold, kWithV, false, DR>(sm, wave, g, n, m_run, l_run, acc, a.n_rep, a.pm + slot * a.n_rep,
                                               a.pl + slot * a.n_rep, a.pacc + slot * a.n_rep * DR);
 }
 
-// Combine the dense partials into the caller's running state, in place.
-// Split-K merge of the operator kernels: one 256-thread workgroup per (batch row, query head).
-// Thread (g, c) owns dims 2c, 2c+1 (D/2 columns) and merges the partial slots g, g+G, g+2G, ...
-// (G = 512/D groups) online, with kDenseMergeBatch slots' loads in flight before it uses any:
-// a running max and sums rescaled under it (e-based units, as the operator state). The groups
-// then combine through LDS with the state already in (m, l, acc). Stats mode merges (m, l)
-// only; the fixed-max modes add the partial sums as they are. A slot whose split held no valid
-// token carries m = -inf and adds nothing; if nothing is valid anywhere the state is left as
-// it was.
-constexpr int kDenseMergeThreads = 256;
-constexpr int kDenseMergeBatch = 8;
+// Split-K merge of the operator kernels into the caller's running state, in place: one workgroup
+// per (batch row, query head). Thread (g, c) owns dims 2c, 2c+1 (D/2 columns) and merges the
+// partial slots g, g+G, g+2G, ... (G = 2 * threads / D groups) online, kU slots' loads in flight
+// before it uses any: a running max and sums rescaled under it (e-based units, as the operator
+// state). The groups then combine through LDS with the state already in (m, l, acc), which loads
+// beside the first partials. Stats mode merges (m, l) only; the fixed-max modes add the partial
+// sums as they are. A slot whose split held no valid token carries m = -inf and adds nothing; if
+// nothing is valid anywhere the state is left as it was.
+//
+// Latency-bound: rounds of dependent loads, not bytes. kU is the smallest of 2, 4, 8 that takes
+// the slots in one round; where 8 per thread do not, the workgroup has 1024 threads.
+// With kU 8 and 256 threads throughout and the state read last: 28/4 heads D 128 fp16, 1024
+// tokens 8.2 us a fold call on the GPU (7.4 now), 32/4 D 64 batch 4 2048 tokens 9.5 (8.4), 6/3 D 8
+// 1024 tokens 10.7 (6.3).
+constexpr int kDenseMergeBatch = 8;  // most slots per thread and round
 
-template <int kMode>
-__global__ __launch_bounds__(kDenseMergeThreads) void dense_merge_kernel(DenseArgs a, float* m, float* l, float* acc,
-                                                                         int d) {
-  __shared__ float sm_m[kDenseMergeThreads];
-  __shared__ float sm_l[kDenseMergeThreads];
-  __shared__ float sm_a[2 * kDenseMergeThreads];
+template <int kMode, int kThreads, int kU>
+__global__ __launch_bounds__(kThreads) void dense_merge_kernel(DenseArgs a, float* m, float* l, float* acc, int d) {
+  __shared__ float sm_m[kThreads];
+  __shared__ float sm_l[kThreads];
+  __shared__ float sm_a[2 * kThreads];
   const int row = blockIdx.x;  // b * hq + qh
   const int b = row / a.hq, qh = row - b * a.hq;
   if (a.active != nullptr && a.active[b] == 0) return;  // whole workgroup: uniform exit
   const int h = qh / a.n_rep, r = qh - h * a.n_rep;
   const size_t slot0 = ((size_t)b * a.hkv + h) * a.n_split;
-  const int cols = d / 2;                          // d is even (8 .. 256)
-  const int groups = kDenseMergeThreads / cols;    // 1 .. 64
+  const int cols = d / 2;                // d is even (8 .. 256)
+  const int groups = kThreads / cols;    // 2 .. 256
   const int g = threadIdx.x / cols, c = threadIdx.x - g * cols;
   constexpr bool kOnline = kMode == kModeFold || kMode == kModeStats;
   constexpr bool kAcc = kMode != kModeStats;
   float mx = kNegInf, ls = 0.f, a0 = 0.f, a1 = 0.f;
+  float m0 = kNegInf, l0 = 0.f;
+  float2 x = {0.f, 0.f};
   const int n = a.n_split;
-  for (int s0 = g; s0 < n; s0 += groups * kDenseMergeBatch) {
-    float pmv[kDenseMergeBatch], plv[kDenseMergeBatch], p0[kDenseMergeBatch], p1[kDenseMergeBatch];
+  for (int s0 = g; s0 < n; s0 += groups * kU) {
+    float pmv[kU], plv[kU], p0[kU], p1[kU];
 #pragma unroll
-    for (int j = 0; j < kDenseMergeBatch; ++j) {
+    for (int j = 0; j < kU; ++j) {
       const int sj = s0 + j * groups;
       const size_t slot = (slot0 + (sj < n ? sj : s0)) * a.n_rep + r;  // past the last slot: re-read s0, weight 0
       pmv[j] = kOnline ? (sj < n ? a.pm[slot] : kNegInf) : 0.f;
@@ -571,8 +666,15 @@ __global__ __launch_bounds__(kDenseMergeThreads) void dense_merge_kernel(DenseAr
         p1[j] = sj < n ? v2.y : 0.f;
       }
     }
+    if (s0 == 0) {  // group 0, first round: the state, which it combines with at the end
+      if constexpr (kOnline) {
+        m0 = m[row];
+        l0 = l[row];
+      }
+      if constexpr (kAcc) x = float2{acc[(size_t)row * d + 2 * c], acc[(size_t)row * d + 2 * c + 1]};
+    }
 #pragma unroll
-    for (int j = 0; j < kDenseMergeBatch; ++j) {
+    for (int j = 0; j < kU; ++j) {
       if constexpr (kOnline) {
         const float mn = fmaxf(mx, pmv[j]);
         if (mn != kNegInf) {
@@ -600,43 +702,36 @@ __global__ __launch_bounds__(kDenseMergeThreads) void dense_merge_kernel(DenseAr
   }
   __syncthreads();
   if (g != 0) return;
+  const int used = min(groups, n);  // groups past the slots hold nothing
   if constexpr (kOnline) {
-    const float m0 = m[row];
     float mf = m0;
-    for (int gg = 0; gg < groups; ++gg) mf = fmaxf(mf, sm_m[gg]);
+    for (int gg = 0; gg < used; ++gg) mf = fmaxf(mf, sm_m[gg]);
     if (mf == kNegInf) return;  // nothing valid anywhere yet: the state stays as it is
     const float w0 = __expf(m0 - mf);
-    float lf = l[row] * w0;
-    float x0 = 0.f, x1 = 0.f;
-    if constexpr (kAcc) {
-      x0 = acc[(size_t)row * d + 2 * c] * w0;
-      x1 = acc[(size_t)row * d + 2 * c + 1] * w0;
-    }
-    for (int gg = 0; gg < groups; ++gg) {
-      if (sm_m[gg] == kNegInf) continue;
-      const float wg = __expf(sm_m[gg] - mf);
+    float lf = l0 * w0;
+    x.x *= w0;
+    x.y *= w0;
+    for (int gg = 0; gg < used; ++gg) {
+      const float wg = __expf(sm_m[gg] - mf);  // an empty group: m = -inf, weight 0, zero sums
       lf += sm_l[gg] * wg;
       if constexpr (kAcc) {
-        x0 += sm_a[gg * d + 2 * c] * wg;
-        x1 += sm_a[gg * d + 2 * c + 1] * wg;
+        x.x += sm_a[gg * d + 2 * c] * wg;
+        x.y += sm_a[gg * d + 2 * c + 1] * wg;
       }
-    }
-    if constexpr (kAcc) {
-      acc[(size_t)row * d + 2 * c] = x0;
-      acc[(size_t)row * d + 2 * c + 1] = x1;
     }
     if (c == 0) {
       m[row] = mf;
       l[row] = lf;
     }
   } else {
-    float x0 = acc[(size_t)row * d + 2 * c], x1 = acc[(size_t)row * d + 2 * c + 1];
-    for (int gg = 0; gg < groups; ++gg) {
-      x0 += sm_a[gg * d + 2 * c];
-      x1 += sm_a[gg * d + 2 * c + 1];
+    for (int gg = 0; gg < used; ++gg) {
+      x.x += sm_a[gg * d + 2 * c];
+      x.y += sm_a[gg * d + 2 * c + 1];
     }
-    acc[(size_t)row * d + 2 * c] = x0;
-    acc[(size_t)row * d + 2 * c + 1] = x1;
+  }
+  if constexpr (kAcc) {
+    acc[(size_t)row * d + 2 * c] = x.x;
+    acc[(size_t)row * d + 2 * c + 1] = x.y;
   }
 }
 
@@ -1412,18 +1507,32 @@ __global__ __launch_bounds__(256) void mass_step_reduce_kernel(const SeqInfo* se
   if (hg == 0 && live) mass_accum[(size_t)sess * accum_stride + blk] = acc;
 }
 
+template <int kMode>
+void launch_dense_merge_t(const DenseArgs& a, int rows, int d, float* m, float* l, float* acc, hipStream_t stream) {
+  const int groups = 512 / d;  // of 256 threads
+  const int per_thread = (a.n_split + groups - 1) / groups;
+  if (per_thread <= 2)
+    dense_merge_kernel<kMode, 256, 2><<<rows, 256, 0, stream>>>(a, m, l, acc, d);
+  else if (per_thread <= 4)
+    dense_merge_kernel<kMode, 256, 4><<<rows, 256, 0, stream>>>(a, m, l, acc, d);
+  else if (per_thread <= kDenseMergeBatch)
+    dense_merge_kernel<kMode, 256, kDenseMergeBatch><<<rows, 256, 0, stream>>>(a, m, l, acc, d);
+  else
+    dense_merge_kernel<kMode, 1024, kDenseMergeBatch><<<rows, 1024, 0, stream>>>(a, m, l, acc, d);
+}
+
 hipError_t launch_dense_merge(const DenseArgs& a, int mode, int batch, int d, float* m, float* l, float* acc,
                               hipStream_t stream) {
-  dim3 mgrid(batch * a.hq);
+  const int rows = batch * a.hq;
   switch (mode) {
     case kModeFold:
-      dense_merge_kernel<kModeFold><<<mgrid, kDenseMergeThreads, 0, stream>>>(a, m, l, acc, d);
+      launch_dense_merge_t<kModeFold>(a, rows, d, m, l, acc, stream);
       break;
     case kModeStats:
-      dense_merge_kernel<kModeStats><<<mgrid, kDenseMergeThreads, 0, stream>>>(a, m, l, acc, d);
+      launch_dense_merge_t<kModeStats>(a, rows, d, m, l, acc, stream);
       break;
     default:
-      dense_merge_kernel<kModeAccumulate><<<mgrid, kDenseMergeThreads, 0, stream>>>(a, m, l, acc, d);
+      launch_dense_merge_t<kModeAccumulate>(a, rows, d, m, l, acc, stream);
       break;
   }
   return hipGetLastError();
@@ -1537,13 +1646,20 @@ bool paged_head_dim_supported(int d) { return d == 16 || d == 32 || d == 64 || d
 
 bool dense_head_dim_supported(int d) { return d == 8 || paged_head_dim_supported(d); }
 
-int dense_wave_tokens(int batch, int hkv, int tc, int tokens_per_block, bool mass) {
+int dense_wave_tokens(int batch, int hkv, int tc, int d, int tokens_per_block, bool mass) {
   // Aim for about 2048 waves over the grid (8 per CU), each folding at least one 16-token tile.
   const long target = 2048;
   const long tiles = (tc + 15) / 16;
   const long rows = (long)batch * hkv;
   long per_wave = (tiles * rows + target - 1) / target;
   if (per_wave < 1) per_wave = 1;
+  // A short chunk of a head stays in one workgroup, which then updates the state itself (one
+  // launch, no partials): up to 256 tokens and 32768 elements of K. Back to back on the GPU, fold /
+  // stats / accumulate, split and merged -> one workgroup: 28/4 heads D 128 fp16, 256 tokens 7.2 /
+  // 6.1 / 6.4 -> 6.2 / 4.6 / 5.4 us, 512 tokens 7.2 / 6.2 / 6.6 -> 8.7 / 6.1 / 7.7; 8/1 D 256 bf16,
+  // 128 tokens 8.2 / 6.3 / 6.3 -> 7.5 / 4.3 / 6.3, 256 tokens 8.3 / 6.3 / 8.1 -> 9.6 / 6.0 / 8.5;
+  // and a launch less on the host either way.
+  if (tc <= 256 && (long)tc * d <= 32768 && per_wave * kWaves < tiles) per_wave = (tiles + kWaves - 1) / kWaves;
   long tokens = per_wave * 16;
   if (mass) {
     const long tpb = tokens_per_block;
@@ -1576,6 +1692,10 @@ hipError_t launch_dense(int dtype, int mode, int d, const DenseLaunch& p, hipStr
   a.block_id_offset = p.block_id_offset;
   a.scale = p.scale;
   a.softcap = p.softcap;
+  const bool direct = p.n_split == 1 && !p.attention_only;
+  a.m_state = direct ? p.m : nullptr;
+  a.l_state = direct ? p.l : nullptr;
+  a.acc_state = direct ? p.acc : nullptr;
   hipError_t e;
   if (p.ev_start != nullptr && (e = hipEventRecord(p.ev_start, stream)) != hipSuccess) return e;
   if (dtype == kF16)
@@ -1586,7 +1706,7 @@ hipError_t launch_dense(int dtype, int mode, int d, const DenseLaunch& p, hipStr
     e = launch_dense_ty<F32>(a, mode, p.batch, d, stream);
   if (e != hipSuccess) return e;
   if (p.ev_stop != nullptr && (e = hipEventRecord(p.ev_stop, stream)) != hipSuccess) return e;
-  if (p.attention_only) return hipSuccess;
+  if (p.attention_only || direct) return hipSuccess;
   return launch_dense_merge(a, mode, p.batch, d, p.m, p.l, p.acc, stream);
 }
 

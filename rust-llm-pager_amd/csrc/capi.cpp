@@ -62,7 +62,7 @@ DensePlan plan_dense(int64_t batch, int64_t hq, int64_t hkv, int64_t tokens, int
   DensePlan p;
   if (tokens <= 0 || batch <= 0) return p;
   const bool mass = mode == PGR_MODE_ACCUMULATE;
-  p.wave_tokens = pgr::dense_wave_tokens((int)batch, (int)hkv, (int)tokens, (int)(mass ? tpb : 16), mass);
+  p.wave_tokens = pgr::dense_wave_tokens((int)batch, (int)hkv, (int)tokens, (int)d, (int)(mass ? tpb : 16), mass);
   const int64_t per_wg = (int64_t)pgr::kWaves * p.wave_tokens;
   p.n_split = (int)((tokens + per_wg - 1) / per_wg);
   const size_t slots = (size_t)batch * hkv * p.n_split;
