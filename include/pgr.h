@@ -36,7 +36,7 @@ extern "C" {
 
 /* ---- library ------------------------------------------------------------------------- */
 
-/* ABI version of this header (increments when an entry point is added or changed); 10. */
+/* ABI version of this header (increments when an entry point is added or changed); 11. */
 int pgr_abi_version(void);
 /* Message of the last failing call on this thread ("" if none). */
 const char* pgr_last_error(void);
@@ -280,6 +280,10 @@ int pgr_kv_set_length(void* kv, int32_t sid, int64_t n_tokens);
  * kv_utils.py:38-61. Synchronous. */
 int pgr_kv_import(void* kv, int32_t sid, int32_t row, int32_t layer, const void* k, const void* v, int64_t n_src,
                   int64_t n_tokens, void* stream);
+/* pgr_kv_import for every layer and row of the session in one call: k, v and n_src are arrays of
+ * num_layers * rows values, entry layer * rows + row. */
+int pgr_kv_import_prompt(void* kv, int32_t sid, const void* const* k, const void* const* v, const int64_t* n_src,
+                         int64_t n_tokens, void* stream);
 /* Reads tokens [0, n_tokens) back into k, v [Hkv, n_tokens, D]. Synchronous.
  * Replaces reconstruct_past_from_store, kv_utils.py:112-178. */
 int pgr_kv_export(void* kv, int32_t sid, int32_t row, int32_t layer, void* k, void* v, int64_t n_tokens, void* stream);

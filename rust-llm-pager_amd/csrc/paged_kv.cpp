@@ -44,20 +44,39 @@ __device__ __forceinline__ VChunk v_chunk(int c, int tpb, int d) {
   return VChunk{h, tile * 16 + 4 * g, dn * n + j};
 }
 
-// One workgroup per block of records: converts tokens of one (row, layer) from the
-// [Hkv, n_src, D] layout into records at dst + slot[i] * rec (zero past n_tokens), or back.
-__global__ void hf_to_records_kernel(const uint16_t* k, const uint16_t* v, int64_t n_src, int64_t n_tokens,
-                                     const int64_t* dst, uint16_t* pool, uint16_t* host, int hkv, int tpb, int d) {
-  // Block i of a [Hkv, n_src, D] tensor pair into its record: dst[i] >= 0 is an HBM pool
-  // slot, dst[i] < 0 the host mirror record -dst[i] - 1 (written in place over the host
-  // link). 16 bytes per store; tokens past n_tokens are zero. K chunk c is 8 dims of one
-  // token row; V chunk c is 2 dims of 4 tokens (the record's transposed V tiles), gathered
-  // from four 4-byte loads.
+// The (layer, row) pairs of one import launch, passed by value in the argument block.
+constexpr int kImportPairs = 64;
+struct ImportBatch {
+  const uint16_t* k[kImportPairs];  // [Hkv, n_src, D]
+  const uint16_t* v[kImportPairs];
+  int64_t n_src[kImportPairs];
+  int32_t layer[kImportPairs];
+  int32_t row[kImportPairs];
+};
+
+// Prompt tokens into records. Workgroup (b, y) converts block b of pair y from the
+// [Hkv, n_src, D] layout: dst[row * blocks + b] >= 0 is an HBM pool slot, < 0 the host mirror
+// record -dst - 1 (written in place over the host link), the same in every layer; bases holds
+// the layers' pools and then their mirrors. 16 bytes per store; tokens past n_tokens are zero.
+// K chunk c is 8 dims of one token row; V chunk c is 2 dims of 4 tokens (the record's transposed
+// V tiles), gathered from four 4-byte loads.
+//
+// One launch per 64 pairs instead of one per pair: a chat prompt's pair is a few microseconds of
+// copying behind as much host time and, with four index buffers, a wait for the fourth launch
+// before: 96 imports (24 layers, 4 sessions of 665 to 889 tokens) took 1.2 ms of a 12-step request,
+// 7.83 ms in all; 6.77 with one launch per session.
+__global__ void hf_to_records_kernel(ImportBatch t, const int64_t* dst, int64_t n_tokens, void* const* bases,
+                                     int num_layers, int hkv, int tpb, int d) {
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   const int64_t b = blockIdx.x;
-  const int64_t di = dst[b];
+  const int y = blockIdx.y;
+  const uint16_t* k = t.k[y];
+  const uint16_t* v = t.v[y];
+  const int64_t n_src = t.n_src[y];
+  const int64_t di = dst[(size_t)t.row[y] * gridDim.x + b];
   const size_t rec = (size_t)2 * hkv * tpb * d;
-  uint16_t* kr = di >= 0 ? pool + (size_t)di * rec : host + (size_t)(-di - 1) * rec;
+  uint16_t* kr = di >= 0 ? static_cast<uint16_t*>(bases[t.layer[y]]) + (size_t)di * rec
+                         : static_cast<uint16_t*>(bases[num_layers + t.layer[y]]) + (size_t)(-di - 1) * rec;
   uint16_t* vr = kr + (size_t)hkv * tpb * d;
   const int cpr = d / 8;  // 16-byte chunks per token row
   const int per = hkv * tpb * cpr;
@@ -683,33 +702,64 @@ int PagedKV::set_length(int sid, int64_t n_tokens) {
 int PagedKV::import_tokens(int sid, int row, int layer, const void* k, const void* v, int64_t n_src, int64_t n_tokens,
                            hipStream_t stream) {
   if (sid < 0 || sid >= (int)sessions_.size() || !sessions_[sid].live) return fail(kErrKey, "unknown session");
+  if (row < 0 || row >= sessions_[sid].rows || layer < 0 || layer >= cfg_.num_layers)
+    return fail(kErrInvalid, "row/layer out of range");
+  return import_pairs(sid, &k, &v, &n_src, layer, 1, row, 1, n_tokens, stream);
+}
+
+int PagedKV::import_prompt(int sid, const void* const* k, const void* const* v, const int64_t* n_src, int64_t n_tokens,
+                           hipStream_t stream) {
+  if (sid < 0 || sid >= (int)sessions_.size() || !sessions_[sid].live) return fail(kErrKey, "unknown session");
+  return import_pairs(sid, k, v, n_src, 0, cfg_.num_layers, 0, sessions_[sid].rows, n_tokens, stream);
+}
+
+// Layers [layer0, layer0 + layers) of rows [row0, row0 + rows): pair i is layer layer0 + i / rows,
+// row row0 + i % rows.
+int PagedKV::import_pairs(int sid, const void* const* k, const void* const* v, const int64_t* n_src, int layer0,
+                          int layers, int row0, int rows, int64_t n_tokens, hipStream_t stream) {
   Session& s = sessions_[sid];
-  if (row < 0 || row >= s.rows || layer < 0 || layer >= cfg_.num_layers) return fail(kErrInvalid, "row/layer out of range");
-  if (n_tokens != s.n_tokens || n_src < n_tokens) return fail(kErrInvalid, "n_tokens must equal the session length");
+  const int pairs = layers * rows;
+  if (n_tokens != s.n_tokens) return fail(kErrInvalid, "n_tokens must equal the session length");
+  for (int i = 0; i < pairs; ++i)
+    if (n_src[i] < n_tokens) return fail(kErrInvalid, "n_tokens must equal the session length");
   if (in_step_) return fail(kErrState, "import during a decode step");
-  if (((uintptr_t)k | (uintptr_t)v) % 16 != 0) return fail(kErrInvalid, "k and v must be 16-byte aligned");
+  for (int i = 0; i < pairs; ++i) {
+    if (!k[i] || !v[i]) return fail(kErrInvalid, "null pointer");
+    if (((uintptr_t)k[i] | (uintptr_t)v[i]) % 16 != 0) return fail(kErrInvalid, "k and v must be 16-byte aligned");
+  }
   const int64_t T = cfg_.tokens_per_block;
   const int64_t nb = (n_tokens + T - 1) / T;
   if (nb == 0) return kOk;
   if (int rc0 = order_after_moves(stream); rc0 != kOk) return rc0;
-  // One launch: resident blocks into their pool slots, host blocks straight into the
-  // pinned mirror through its device mapping.
+  // Resident blocks go into their pool slots, host blocks straight into the pinned mirror through
+  // its device mapping.
   IndexBuf* ib = nullptr;
-  int rc = acquire_index_buf((size_t)nb, &ib);
+  int rc = acquire_index_buf((size_t)(nb * rows), &ib);
   if (rc != kOk) return rc;
-  for (int64_t b = 0; b < nb; ++b) {
-    const int32_t sl = s.slot[b * s.rows + row];
-    ib->host[b] = sl >= 0 ? (int64_t)sl : -(s.row[row].host_off + b) - 1;
+  for (int r = 0; r < rows; ++r)
+    for (int64_t b = 0; b < nb; ++b) {
+      const int32_t sl = s.slot[b * s.rows + row0 + r];
+      ib->host[r * nb + b] = sl >= 0 ? (int64_t)sl : -(s.row[row0 + r].host_off + b) - 1;
+    }
+  for (int at = 0; at < pairs; at += kImportPairs) {
+    const int n = std::min(kImportPairs, pairs - at);
+    ImportBatch t{};
+    for (int i = 0; i < n; ++i) {
+      t.k[i] = static_cast<const uint16_t*>(k[at + i]);
+      t.v[i] = static_cast<const uint16_t*>(v[at + i]);
+      t.n_src[i] = n_src[at + i];
+      t.layer[i] = layer0 + (at + i) / rows;
+      t.row[i] = (at + i) % rows;
+    }
+    hf_to_records_kernel<<<dim3((unsigned)nb, (unsigned)n), 256, 0, stream>>>(
+        t, ib->dev, n_tokens, bases_dev_, cfg_.num_layers, cfg_.kv_heads, (int)T, cfg_.head_dim);
+    PGR_HIP(hipGetLastError());
   }
-  hf_to_records_kernel<<<(unsigned)nb, 256, 0, stream>>>(
-      static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), n_src, n_tokens, ib->dev,
-      static_cast<uint16_t*>(pool_[layer]), static_cast<uint16_t*>(host_dev_[layer]), cfg_.kv_heads, (int)T,
-      cfg_.head_dim);
-  PGR_HIP(hipGetLastError());
   PGR_HIP(hipEventRecord(ib->done, stream));
   ib->pending = true;
-  for (int64_t b = 0; b < nb; ++b)
-    if (s.slot[b * s.rows + row] < 0) s.host_valid[b * s.rows + row] = 1;
+  for (int r = row0; r < row0 + rows; ++r)
+    for (int64_t b = 0; b < nb; ++b)
+      if (s.slot[b * s.rows + r] < 0) s.host_valid[b * s.rows + r] = 1;
   return kOk;
 }
 

@@ -148,6 +148,10 @@ class PagedKV {
   int set_length(int sid, int64_t n_tokens);
   int import_tokens(int sid, int row, int layer, const void* k, const void* v, int64_t n_src, int64_t n_tokens,
                     hipStream_t stream);
+  // The same for every layer and row of the session at once: k, v and n_src hold num_layers * rows
+  // values, layer by layer.
+  int import_prompt(int sid, const void* const* k, const void* const* v, const int64_t* n_src, int64_t n_tokens,
+                    hipStream_t stream);
   // Read back tokens [0, n) of one (session, row, layer) into k, v [Hkv, n, D] (device).
   int export_tokens(int sid, int row, int layer, void* k, void* v, int64_t n_tokens, hipStream_t stream);
 
@@ -289,6 +293,8 @@ class PagedKV {
   };
   static constexpr int kIndexBufs = 4;
   int acquire_index_buf(size_t n, IndexBuf** out);
+  int import_pairs(int sid, const void* const* k, const void* const* v, const int64_t* n_src, int layer0, int layers,
+                   int row0, int rows, int64_t n_tokens, hipStream_t stream);
   // Copies records (from, to) pairs for every layer in one launch; tables 0 (HBM pool) or
   // num_layers (host mirror) select source and destination. Clears `pairs`.
   int launch_copies(std::vector<int64_t>& pairs, int src_tbl, int dst_tbl, hipStream_t stream);

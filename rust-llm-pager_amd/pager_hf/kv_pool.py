@@ -163,6 +163,32 @@ class NativeKVPool:
         self._call("import", self.lib.pgr_kv_import, sid, row, layer, k.data_ptr(), v.data_ptr(), k.shape[1],
                    n_tokens, self._stream())
 
+    def import_prompt(self, sid: int, rows: int, keys, values, n_tokens: int) -> None:
+        """Every layer and row at once: keys[layer][row], values[layer][row] as for import_tokens."""
+        held = []  # the tensors the launches read
+        kp, vp, n_src = [], [], []
+        for layer in range(self.num_layers):
+            k, v = keys[layer], values[layer]
+            if (type(k) is torch.Tensor and type(v) is torch.Tensor and k.dim() == 4 and v.dim() == 4
+                    and k.shape[0] >= rows and v.shape[0] >= rows and k.is_contiguous() and v.is_contiguous()):
+                self._check_kv(k, v)  # rows of one contiguous tensor
+                ks, vs = k.stride(0) * k.element_size(), v.stride(0) * v.element_size()
+                k0, v0 = k.data_ptr(), v.data_ptr()
+                kp.extend(k0 + r * ks for r in range(rows))
+                vp.extend(v0 + r * vs for r in range(rows))
+                n_src.extend([k.shape[2]] * rows)
+                continue
+            for row in range(rows):
+                kr, vr = k[row].contiguous(), v[row].contiguous()
+                self._check_kv(kr, vr)
+                held.append((kr, vr))
+                kp.append(kr.data_ptr())
+                vp.append(vr.data_ptr())
+                n_src.append(kr.shape[1])
+        n = len(kp)
+        self._call("import", self.lib.pgr_kv_import_prompt, sid, (ctypes.c_void_p * n)(*kp), (ctypes.c_void_p * n)(*vp),
+                   (ctypes.c_int64 * n)(*n_src), n_tokens, self._stream())
+
     def export_tokens(self, sid: int, row: int, layer: int, n_tokens: int):
         k = torch.empty((self.num_kv_heads, n_tokens, self.head_dim), dtype=self.dtype, device=self.device)
         v = torch.empty_like(k)

@@ -188,9 +188,7 @@ class PagedDecoder:
             if host_ids:  # prompt blocks placed host-side count as offloaded (kv_block_store.py:101-108)
                 self._warn_ram_usage(host_ids[-1])
         if n_tokens:
-            for layer in range(self.num_layers):
-                for row in range(s.rows):
-                    self.pool.import_tokens(sid, row, layer, keys[layer][row], values[layer][row], n_tokens)
+            self.pool.import_prompt(sid, s.rows, keys, values, n_tokens)
         return moves
 
     def _warn_ram_usage(self, block_id: int) -> None:
