@@ -1265,11 +1265,15 @@ __global__ __launch_bounds__(256) void paged_merge_kernel(const SeqInfo* __restr
   const int P = si->partial_count;  // P >= 1: every sequence has a work item
   // Deferred mass: the thread's first block's entries, loaded beside the partials.
   const size_t mass_row = ((size_t)seq * hq + qh) * a.mass_stride;
-  const int mass_b0 = si->mass_lo + tid, n_mass = a.mass_w != nullptr ? si->n_mass : 0;
+  int mass_b0 = 0, n_mass = 0;
   float mass_m0 = 0.f, mass_s0 = 0.f;
-  if (mass_b0 < n_mass) {
-    mass_m0 = a.mass_m[mass_row + mass_b0];
-    mass_s0 = a.mass_s[mass_row + mass_b0];
+  if (a.mass_w != nullptr) {
+    mass_b0 = si->mass_lo + tid;
+    n_mass = si->n_mass;
+    if (mass_b0 < n_mass) {
+      mass_m0 = a.mass_m[mass_row + mass_b0];
+      mass_s0 = a.mass_s[mass_row + mass_b0];
+    }
   }
   const int h = qh / n_rep;
   const size_t kv_row = ((size_t)seq * hkv + h) * D;
