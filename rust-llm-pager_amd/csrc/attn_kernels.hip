@@ -1196,29 +1196,34 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const WorkItem* __restr
 // ---------------------------------------------------------------------------------------
 // Split-K merge: one workgroup per (sequence, query head). Thread (g, c) owns output dims
 // 2c, 2c+1 and merges the partial slots g, g+G, g+2G, ... online (running max, rescaled
-// sums), G = 512 / D thread groups; the groups are then combined through LDS together with
-// the current token (score q.k_new, weight 2^(x - m), P rounded like every other P), and the
-// output and the final (m, l) for the mass pass are written. The kernel is latency-bound:
+// sums), G = 2 * threads / D thread groups; the groups are then combined through LDS together
+// with the current token (score q.k_new, weight 2^(x - m), P rounded like every other P), and
+// the output and the final (m, l) for the mass pass are written. The kernel is latency-bound:
 // each thread issues a whole batch of partial loads before using any of them (a load past
 // the last partial re-reads it and is weighted 0).
 //
-// kU, slots per thread and batch: the smallest of 1, 2, 4, 8, 16 whose one batch covers every
-// slot range of the step (16, in several batches, beyond that and for packed slots). Slots past
-// a sequence's count add exact zeros, so the sums do not depend on it; fewer of them are loads
-// and exponentials the kernel does without. Per layer (attention and merge), 64 sequences of 93
-// to 2038 tokens at head dim 128 (14 slots at most): 25.6 us with 16 slots per thread, 23.3 with
-// 4; with block mass 27.2 and 24.7. 8 sequences at head dim 64 (74 slots): 16 per thread still.
+// kU, slots per thread and batch: the smallest of 1, 2, 4, 6, 8, 10, 12, 16 whose one batch covers
+// every slot range of the step. Slots past a sequence's count add exact zeros, so the sums do not
+// depend on it; fewer of them are loads that the batch does not queue behind. Beyond 16 per
+// thread the workgroup has 1024 threads and batches of 8; packed slots, whose counts differ too
+// much for one range, keep 16 in 256 threads. Per layer (attention and merge), against 16 per
+// thread in 256 threads: 64 sequences of 93 to 2038 tokens at head dim 128 (14 slots at most)
+// 25.6 -> 23.3 us, with block mass 27.2 -> 24.7; 8 sequences up to 28770 tokens at head dim 64
+// (74 slots) 20.0 -> 19.6, with block mass 22.25 -> 21.85; two of 16384 at 8/1 heads, head dim 256
+// (256 slots) 16.6 -> 15.2. (512 threads with 6 slots took 19.5 and 21.3 at the 8 sequences, but add
+// the slots in another order, which turns a 0.004 logit gap of the 8192-token TinyLlama run into
+// another token.)
 constexpr int kMergeBatch = 16;
 
 // The leading arguments are preloaded into SGPRs (as in paged_attn_kernel): the partial loads
 // of the first batch depend on nothing else, and go out before the plan's SeqInfo arrives.
-template <class Ty, int D, int kU>
-__global__ __launch_bounds__(256) void paged_merge_kernel(const SeqInfo* __restrict__ seqs, const float* pm0,
+template <class Ty, int D, int kU, int kThreads>
+__global__ __launch_bounds__(kThreads) void paged_merge_kernel(const SeqInfo* __restrict__ seqs, const float* pm0,
                                                           const float* pl0, const float* pacc0,
                                                           int partial_stride, int hq, int n_rep, int hkv,
                                                           PagedArgs a) {
   constexpr int kLanes = D / 2;          // threads per partial group (two dims each)
-  constexpr int G = 256 / kLanes;        // partial groups
+  constexpr int G = kThreads / kLanes;   // partial groups
   constexpr int kRed = kLanes < kWaveSize ? kLanes : kWaveSize;  // lanes of group 0 per wave
   __shared__ float m_s[G], l_s[G];
   __shared__ float acc_s[G][D];
@@ -1388,7 +1393,7 @@ __global__ __launch_bounds__(256) void paged_merge_kernel(const SeqInfo* __restr
   __syncthreads();
   const float mfin = fin_s[0], lfin = fin_s[1];
   if (mass_b0 < n_mass) a.mass_w[mass_row + mass_b0] = mass_s0 * __builtin_amdgcn_exp2f(mass_m0 - mfin) / lfin;
-  for (int b = mass_b0 + 256; b < n_mass; b += 256)
+  for (int b = mass_b0 + kThreads; b < n_mass; b += kThreads)
     a.mass_w[mass_row + b] = a.mass_s[mass_row + b] * __builtin_amdgcn_exp2f(a.mass_m[mass_row + b] - mfin) / lfin;
 }
 
@@ -1607,21 +1612,35 @@ hipError_t launch_paged_d(const PagedArgs& a, int d, int n_work, bool mass, hipS
   }
 }
 
+template <class Ty, int D, int kU, int kThreads>
+void launch_merge_u(const PagedArgs& a, int stride, dim3 grid, hipStream_t stream) {
+  paged_merge_kernel<Ty, D, kU, kThreads>
+      <<<grid, kThreads, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep, a.hkv, a);
+}
+
 template <class Ty, int D>
 void launch_merge_t(const PagedArgs& a, int stride, dim3 grid, hipStream_t stream) {
-  constexpr int G = 512 / D;  // thread groups of the kernel
-  const int per_group = stride > 0 ? (stride + G - 1) / G : kMergeBatch;
-  if (per_group <= 1)
-    paged_merge_kernel<Ty, D, 1><<<grid, 256, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep, a.hkv, a);
-  else if (per_group <= 2)
-    paged_merge_kernel<Ty, D, 2><<<grid, 256, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep, a.hkv, a);
-  else if (per_group <= 4)
-    paged_merge_kernel<Ty, D, 4><<<grid, 256, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep, a.hkv, a);
-  else if (per_group <= 8)
-    paged_merge_kernel<Ty, D, 8><<<grid, 256, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep, a.hkv, a);
+  constexpr int G = 512 / D;  // thread groups of a 256-thread workgroup
+  if (stride == 0) return launch_merge_u<Ty, D, kMergeBatch, 256>(a, stride, grid, stream);  // packed slots
+  const int n = (stride + G - 1) / G;
+  if (n <= 1)
+    launch_merge_u<Ty, D, 1, 256>(a, stride, grid, stream);
+  else if (n <= 2)
+    launch_merge_u<Ty, D, 2, 256>(a, stride, grid, stream);
+  else if (n <= 4)
+    launch_merge_u<Ty, D, 4, 256>(a, stride, grid, stream);
+  else if (n <= 6)
+    launch_merge_u<Ty, D, 6, 256>(a, stride, grid, stream);
+  else if (n <= 8)
+    launch_merge_u<Ty, D, 8, 256>(a, stride, grid, stream);
+  else if (n <= 10)
+    launch_merge_u<Ty, D, 10, 256>(a, stride, grid, stream);
+  else if (n <= 12)
+    launch_merge_u<Ty, D, 12, 256>(a, stride, grid, stream);
+  else if (n <= kMergeBatch)
+    launch_merge_u<Ty, D, kMergeBatch, 256>(a, stride, grid, stream);
   else
-    paged_merge_kernel<Ty, D, kMergeBatch><<<grid, 256, 0, stream>>>(a.seqs, a.pm, a.pl, a.pacc, stride, a.hq, a.n_rep,
-                                                                     a.hkv, a);
+    launch_merge_u<Ty, D, 8, 1024>(a, stride, grid, stream);
 }
 
 template <class Ty>

@@ -20,6 +20,9 @@ pytestmark = pytest.mark.gpu
 
 CONTEXTS = {
     "single": [3100],
+    "6 slots": [1500],
+    "10 slots": [2300],
+    "12 slots": [2800],
     "few": [1, 1700, 40, 900],
     "many": [15, 16, 17, 33, 700, 95, 96, 97, 300, 64, 5, 128, 31, 32, 511, 210, 47, 48, 49, 1000],
 }
@@ -30,7 +33,7 @@ CONTEXTS = {
 @pytest.mark.parametrize("hq,hkv,d,tpb,dtype", [
     (14, 2, 64, 32, torch.float16), (12, 2, 128, 16, torch.bfloat16), (16, 1, 16, 64, torch.float16),
     (8, 1, 256, 32, torch.bfloat16), (4, 2, 256, 64, torch.float16), (6, 3, 32, 48, torch.float16),
-    (4, 1, 64, 128, torch.float16),
+    (4, 1, 64, 128, torch.float16), (8, 1, 256, 16, torch.bfloat16),
 ])
 def test_uneven_sequences_match_the_oracle(hq, hkv, d, tpb, dtype, policy, contexts):
     print(f"uneven sequences: {contexts} {policy} {hq}/{hkv} d={d} tpb={tpb} {dtype}", flush=True)
