@@ -156,10 +156,8 @@ class NativeKVPool:
         self._call("set_length", self.lib.pgr_kv_set_length, sid, n_tokens)
 
     def import_tokens(self, sid: int, row: int, layer: int, k: torch.Tensor, v: torch.Tensor, n_tokens: int) -> None:
-        """k, v [Hkv, n_src, D] on this device (n_src >= n_tokens)."""
-        k = k.contiguous()
-        v = v.contiguous()
-        self._check_kv(k, v)
+        """k, v [Hkv, n_src, D] on this device (n_src >= n_tokens each)."""
+        k, v = self._row_kv(k, v, n_tokens)
         self._call("import", self.lib.pgr_kv_import, sid, row, layer, k.data_ptr(), v.data_ptr(), k.shape[1],
                    n_tokens, self._stream())
 
@@ -170,8 +168,11 @@ class NativeKVPool:
         for layer in range(self.num_layers):
             k, v = keys[layer], values[layer]
             if (type(k) is torch.Tensor and type(v) is torch.Tensor and k.dim() == 4 and v.dim() == 4
-                    and k.shape[0] >= rows and v.shape[0] >= rows and k.is_contiguous() and v.is_contiguous()):
+                    and k.shape[0] >= rows and v.shape[0] >= rows and k.shape[2] == v.shape[2]
+                    and k.is_contiguous() and v.is_contiguous()):
                 self._check_kv(k, v)  # rows of one contiguous tensor
+                self._check_heads(k.shape[1:])
+                self._check_heads(v.shape[1:])
                 ks, vs = k.stride(0) * k.element_size(), v.stride(0) * v.element_size()
                 k0, v0 = k.data_ptr(), v.data_ptr()
                 kp.extend(k0 + r * ks for r in range(rows))
@@ -179,8 +180,7 @@ class NativeKVPool:
                 n_src.extend([k.shape[2]] * rows)
                 continue
             for row in range(rows):
-                kr, vr = k[row].contiguous(), v[row].contiguous()
-                self._check_kv(kr, vr)
+                kr, vr = self._row_kv(k[row], v[row], n_tokens)
                 held.append((kr, vr))
                 kp.append(kr.data_ptr())
                 vp.append(vr.data_ptr())
@@ -217,6 +217,23 @@ class NativeKVPool:
             raise ValueError(f"tensors must be on {self.device}")
         if k.dtype != self.dtype or v.dtype != self.dtype:
             raise TypeError(f"tensors must be {self.dtype}")
+
+    def _check_heads(self, shape: torch.Size) -> None:
+        """One row of a prompt: the kernel reads [Hkv, n_src, D] by this pool's Hkv and D."""
+        if len(shape) != 3 or shape[0] != self.num_kv_heads or shape[2] != self.head_dim:
+            raise ValueError(f"a row's keys and values must be [{self.num_kv_heads}, tokens, {self.head_dim}], "
+                             f"got {list(shape)}")
+
+    def _row_kv(self, k: torch.Tensor, v: torch.Tensor, n_tokens: int) -> tuple[torch.Tensor, torch.Tensor]:
+        """One row's K and V as the import reads them: contiguous, of this pool's shape and of one length."""
+        self._check_kv(k, v)
+        self._check_heads(k.shape)
+        self._check_heads(v.shape)
+        if k.shape[1] != v.shape[1]:
+            if min(k.shape[1], v.shape[1]) < n_tokens:
+                raise ValueError(f"keys of {k.shape[1]} and values of {v.shape[1]} tokens for {n_tokens}")
+            k, v = k[:, :n_tokens], v[:, :n_tokens]
+        return k.contiguous(), v.contiguous()
 
     # -- placement -----------------------------------------------------------------------
     def apply_tiers(self, sid: int, tiers) -> tuple[list[int], list[int], int, int]:
