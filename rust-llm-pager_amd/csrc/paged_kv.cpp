@@ -741,7 +741,8 @@ int PagedKV::import_pairs(int sid, const void* const* k, const void* const* v, c
       const int32_t sl = s.slot[b * s.rows + row0 + r];
       ib->host[r * nb + b] = sl >= 0 ? (int64_t)sl : -(s.row[row0 + r].host_off + b) - 1;
     }
-  for (int at = 0; at < pairs; at += kImportPairs) {
+  hipError_t launched = hipSuccess;
+  for (int at = 0; at < pairs && launched == hipSuccess; at += kImportPairs) {
     const int n = std::min(kImportPairs, pairs - at);
     ImportBatch t{};
     for (int i = 0; i < n; ++i) {
@@ -753,10 +754,12 @@ int PagedKV::import_pairs(int sid, const void* const* k, const void* const* v, c
     }
     hf_to_records_kernel<<<dim3((unsigned)nb, (unsigned)n), 256, 0, stream>>>(
         t, ib->dev, n_tokens, bases_dev_, cfg_.num_layers, cfg_.kv_heads, (int)T, cfg_.head_dim);
-    PGR_HIP(hipGetLastError());
+    launched = hipGetLastError();
   }
+  // Batches before a failed one still read the index buffer: its next user waits for them too.
   PGR_HIP(hipEventRecord(ib->done, stream));
   ib->pending = true;
+  PGR_HIP(launched);
   for (int r = row0; r < row0 + rows; ++r)
     for (int64_t b = 0; b < nb; ++b)
       if (s.slot[b * s.rows + r] < 0) s.host_valid[b * s.rows + r] = 1;

@@ -2,6 +2,8 @@
 form of the caller's K/V, read back bit for bit."""
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -58,4 +60,29 @@ def test_prompt_import_refuses_what_a_single_import_does():
     with pytest.raises(ValueError):
         dec.pool.import_prompt(sid, 2, good, good, 41)
     dec.pool.import_prompt(sid, 2, good, good, 40)
+    dec.pool.close()
+
+
+def test_index_buffer_of_a_failed_import_is_not_reused_before_the_gpu_has_read_it():
+    """An import that reports an error after some of its launches went out: the buffer of block
+    indices those launches read comes round again (four buffers) only once they have run."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    layers, n = 65, 40  # two launches
+    dec = PagedDecoder(num_layers=layers, num_query_heads=2, num_kv_heads=1, head_dim=16, tokens_per_block=32,
+                       dtype=torch.float16, device="cuda", pool_blocks=16, host_blocks=16, staging_blocks=16)
+    sids = [dec.add_session(capacity_tokens=128, rows=1, vram_budget=4 * MIB16, ram_budget=1 << 40) for _ in range(2)]
+    kv = [torch.zeros(1, 1, n, 16, device="cuda").half() for _ in range(layers)]
+    for sid in sids:
+        dec.prefill(sid, kv, kv, n)
+    torch.cuda.synchronize()
+    torch.cuda._sleep(10_000_000)  # about 100 ms ahead of the imports
+    done = torch.cuda.Event()
+    done.record()
+    assert hip.hipSetDevice(9999) != 0  # leaves an error for the import's launch check to find
+    with pytest.raises(RuntimeError):
+        dec.pool.import_prompt(sids[0], 1, kv, kv, n)
+    assert not done.query()
+    for _ in range(4):
+        dec.pool.import_prompt(sids[1], 1, kv, kv, n)
+    assert done.query()
     dec.pool.close()
