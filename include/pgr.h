@@ -277,11 +277,13 @@ int pgr_kv_reorder_rows(void* kv, int32_t sid, const int32_t* src_rows, int32_t 
 int pgr_kv_set_length(void* kv, int32_t sid, int64_t n_tokens);
 /* Writes tokens [0, n_tokens) of (sid, row, layer) from k, v [Hkv, n_src, D] (device).
  * Replaces _build_initial_store + real_past_to_blocks, paged_model.py:1183-1192 and
- * kv_utils.py:38-61. Synchronous. */
+ * kv_utils.py:38-61. Queued on `stream`, as every call not marked otherwise: k and v must stay
+ * as they are until the stream has passed the call. */
 int pgr_kv_import(void* kv, int32_t sid, int32_t row, int32_t layer, const void* k, const void* v, int64_t n_src,
                   int64_t n_tokens, void* stream);
 /* pgr_kv_import for every layer and row of the session in one call: k, v and n_src are arrays of
- * num_layers * rows values, entry layer * rows + row. */
+ * num_layers * rows values, entry layer * rows + row. The arrays are read during the call, the
+ * K/V they point to by the queued launches. */
 int pgr_kv_import_prompt(void* kv, int32_t sid, const void* const* k, const void* const* v, const int64_t* n_src,
                          int64_t n_tokens, void* stream);
 /* Reads tokens [0, n_tokens) back into k, v [Hkv, n_tokens, D]. Synchronous.
