@@ -3,7 +3,7 @@
 //
 // Each function checks that its arguments are what the kernels take as they are (exact
 // torch.Tensor objects without functorch, functionalization or lazy-bit keys, one GPU, one
-// dtype, contiguous, matching shapes), allocates the workspace or outputs from torch's caching
+// dtype, contiguous, matching shapes), allocates the workspace or outputs from torch's current
 // allocator, and calls the C entry point of libpgr.so. It returns the entry point's status, or
 // None where any check fails: the caller then runs its general Python path, which converts,
 // copies or refuses as it always has. So this file decides nothing but speed: checks in Python,
@@ -16,6 +16,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/detail/CUDAHooksInterface.h>
 #include <c10/core/Allocator.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -174,8 +175,11 @@ PyObject* run(Call& c, int mode, int64_t tpb, F launch) {
   {
     const c10::DeviceGuard guard(c.dev);
     const size_t bytes = g_workspace_bytes(c.b, c.hq, c.hkv, c.tc, c.d, mode, tpb);
-    // Freed on return, behind this stream's work, as a tensor of this size would be.
-    const c10::DataPtr ws = c10::GetAllocator(c10::DeviceType::CUDA)->allocate(bytes ? bytes : 1);
+    // Freed on return, behind this stream's work, as a tensor of this size would be, and from the
+    // allocator that torch.empty uses (c10::GetAllocator is the native one also where
+    // torch.cuda.memory.change_current_allocator has put another in its place).
+    const c10::DataPtr ws =
+        at::detail::getCUDAHooks().getCUDADeviceAllocator()->allocate(bytes ? bytes : 1);
     Py_BEGIN_ALLOW_THREADS;
     rc = launch(ws.get(), bytes);
     Py_END_ALLOW_THREADS;

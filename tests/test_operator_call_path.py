@@ -6,6 +6,10 @@ same kernels on the same values), and what one refuses the other refuses with th
 """
 from __future__ import annotations
 
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -165,6 +169,55 @@ def test_functorch_and_modes_take_the_general_path():
 
     torch.func.vmap(probe)(x)
     assert taken == [None]
+
+
+_ALLOCATOR_C = """
+#include <stddef.h>
+#include <sys/types.h>
+static int (*dev_malloc)(void**, size_t);
+static int (*dev_free)(void*);
+long sizes[1024];
+int n_sizes;
+void set_functions(void* m, void* f) { dev_malloc = m; dev_free = f; }
+void* dev_alloc(ssize_t size, int device, void* stream) {
+  void* p = 0;
+  if (n_sizes < 1024) sizes[n_sizes++] = size;
+  return dev_malloc(&p, size) == 0 ? p : 0;
+}
+void dev_release(void* p, ssize_t size, int device, void* stream) { dev_free(p); }
+"""
+
+_ALLOCATOR_PY = """
+import ctypes, sys
+import torch
+so, hip = ctypes.CDLL(sys.argv[1]), ctypes.CDLL("libamdhip64.so")
+so.set_functions(ctypes.cast(hip.hipMalloc, ctypes.c_void_p), ctypes.cast(hip.hipFree, ctypes.c_void_p))
+torch.cuda.memory.change_current_allocator(
+    torch.cuda.memory.CUDAPluggableAllocator(sys.argv[1], "dev_alloc", "dev_release"))
+from pager_hf import _native as N
+from pager_hf import streaming_attention as S
+q, k = torch.randn(1, 4, 64).half().cuda(), torch.randn(1, 2, 3001, 64).half().cuda()
+m, l, acc = S.streaming_attention_state_init(1, 4, 64, q.device)
+S.streaming_attention_step(q, k, k, m, l, acc)
+out = S.streaming_attention_finalize(acc, l, torch.float32)
+p = torch.softmax(q.float().view(2, 2, 64) @ k[0].float().transpose(1, 2).contiguous() / 8, -1)
+assert torch.allclose(out.view(2, 2, 64), p @ k[0].float(), atol=2e-3)
+nbytes = N.lib().pgr_attn_workspace_bytes(1, 4, 2, 3001, 64, N.nat.MODE_FOLD, 16)
+sizes = list((ctypes.c_long * 1024).in_dll(so, "sizes"))[: ctypes.c_int.in_dll(so, "n_sizes").value]
+assert nbytes in sizes, (nbytes, sizes)
+print("workspace from the program's allocator")
+"""
+
+
+@gpu
+def test_workspace_comes_from_the_allocator_that_the_program_set(tmp_path):
+    """change_current_allocator must run before any GPU allocation, so in a process of its own."""
+    src, so = tmp_path / "allocator.c", tmp_path / "allocator.so"
+    src.write_text(_ALLOCATOR_C)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    res = subprocess.run([sys.executable, "-c", _ALLOCATOR_PY, str(so)], capture_output=True, text=True, timeout=100,
+                         env=dict(os.environ, PYTHONPATH=os.pathsep.join(sys.path)))
+    assert res.returncode == 0 and "workspace from" in res.stdout, res.stdout + res.stderr
 
 
 def test_ordinary_cpu_tensors_are_left_to_the_general_path():
