@@ -36,7 +36,7 @@ extern "C" {
 
 /* ---- library ------------------------------------------------------------------------- */
 
-/* ABI version of this header (increments when an entry point is added or changed); 11. */
+/* ABI version of this header (increments when an entry point is added or changed); 12. */
 int pgr_abi_version(void);
 /* Message of the last failing call on this thread ("" if none). */
 const char* pgr_last_error(void);
@@ -286,6 +286,10 @@ int pgr_kv_import(void* kv, int32_t sid, int32_t row, int32_t layer, const void*
  * K/V they point to by the queued launches. */
 int pgr_kv_import_prompt(void* kv, int32_t sid, const void* const* k, const void* const* v, const int64_t* n_src,
                          int64_t n_tokens, void* stream);
+/* The same for layers [layer0, layer0 + n_layers) only (n_layers * rows values), for callers that
+ * have one part of a prompt in hand at a time. */
+int pgr_kv_import_layers(void* kv, int32_t sid, int32_t layer0, int32_t n_layers, const void* const* k,
+                         const void* const* v, const int64_t* n_src, int64_t n_tokens, void* stream);
 /* Reads tokens [0, n_tokens) back into k, v [Hkv, n_tokens, D]. Synchronous.
  * Replaces reconstruct_past_from_store, kv_utils.py:112-178. */
 int pgr_kv_export(void* kv, int32_t sid, int32_t row, int32_t layer, void* k, void* v, int64_t n_tokens, void* stream);

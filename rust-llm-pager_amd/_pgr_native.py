@@ -36,7 +36,7 @@ STREAM_DIRECT = 0
 STREAM_STAGED = 1
 STREAM_MIRROR = 2
 
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 c_i32, c_i64, c_u8, c_u32, c_u64 = ctypes.c_int32, ctypes.c_int64, ctypes.c_uint8, ctypes.c_uint32, ctypes.c_uint64
 c_f32, c_f64, c_size, c_vp = ctypes.c_float, ctypes.c_double, ctypes.c_size_t, ctypes.c_void_p
@@ -159,6 +159,7 @@ SIGNATURES: dict[str, tuple] = {
     "pgr_kv_set_length": (ctypes.c_int, [c_vp, c_i32, c_i64]),
     "pgr_kv_import": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_vp, c_vp, c_i64, c_i64, c_vp]),
     "pgr_kv_import_prompt": (ctypes.c_int, [c_vp, c_i32, P(c_vp), P(c_vp), P(c_i64), c_i64, c_vp]),
+    "pgr_kv_import_layers": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, P(c_vp), P(c_vp), P(c_i64), c_i64, c_vp]),
     "pgr_kv_export": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_vp, c_vp, c_i64, c_vp]),
     "pgr_kv_put_block": (ctypes.c_int, [c_vp, c_i32, c_i64, c_vp, c_vp, c_vp]),
     "pgr_kv_get_block": (ctypes.c_int, [c_vp, c_i32, c_i64, c_vp, c_vp, c_vp]),

@@ -260,7 +260,7 @@ int kv_rc(pgr::PagedKV* kv, int rc) {
 
 extern "C" {
 
-int pgr_abi_version(void) { return 11; }
+int pgr_abi_version(void) { return 12; }
 
 const char* pgr_last_error(void) { return g_last_error.c_str(); }
 
@@ -701,7 +701,19 @@ int pgr_kv_import_prompt(void* kv, int32_t sid, const void* const* k, const void
                          int64_t n_tokens, void* stream) {
   try {
     if (!kv || !k || !v || !n_src) return set_err(pgr::kErrInvalid, "null pointer");
-    return kv_rc(kv_of(kv), kv_of(kv)->import_prompt(sid, k, v, n_src, n_tokens, as_stream(stream)));
+    return kv_rc(kv_of(kv), kv_of(kv)->import_layers(sid, 0, kv_of(kv)->cfg().num_layers, k, v, n_src, n_tokens,
+                                                     as_stream(stream)));
+  } catch (...) {
+    return exception_status();
+  }
+}
+
+int pgr_kv_import_layers(void* kv, int32_t sid, int32_t layer0, int32_t n_layers, const void* const* k,
+                         const void* const* v, const int64_t* n_src, int64_t n_tokens, void* stream) {
+  try {
+    if (!kv || !k || !v || !n_src) return set_err(pgr::kErrInvalid, "null pointer");
+    return kv_rc(kv_of(kv),
+                 kv_of(kv)->import_layers(sid, layer0, n_layers, k, v, n_src, n_tokens, as_stream(stream)));
   } catch (...) {
     return exception_status();
   }

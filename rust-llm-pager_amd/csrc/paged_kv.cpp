@@ -707,10 +707,12 @@ int PagedKV::import_tokens(int sid, int row, int layer, const void* k, const voi
   return import_pairs(sid, &k, &v, &n_src, layer, 1, row, 1, n_tokens, stream);
 }
 
-int PagedKV::import_prompt(int sid, const void* const* k, const void* const* v, const int64_t* n_src, int64_t n_tokens,
-                           hipStream_t stream) {
+int PagedKV::import_layers(int sid, int layer0, int n_layers, const void* const* k, const void* const* v,
+                           const int64_t* n_src, int64_t n_tokens, hipStream_t stream) {
   if (sid < 0 || sid >= (int)sessions_.size() || !sessions_[sid].live) return fail(kErrKey, "unknown session");
-  return import_pairs(sid, k, v, n_src, 0, cfg_.num_layers, 0, sessions_[sid].rows, n_tokens, stream);
+  if (layer0 < 0 || n_layers < 0 || layer0 > cfg_.num_layers - n_layers)
+    return fail(kErrInvalid, "row/layer out of range");
+  return import_pairs(sid, k, v, n_src, layer0, n_layers, 0, sessions_[sid].rows, n_tokens, stream);
 }
 
 // Layers [layer0, layer0 + layers) of rows [row0, row0 + rows): pair i is layer layer0 + i / rows,

@@ -148,10 +148,10 @@ class PagedKV {
   int set_length(int sid, int64_t n_tokens);
   int import_tokens(int sid, int row, int layer, const void* k, const void* v, int64_t n_src, int64_t n_tokens,
                     hipStream_t stream);
-  // The same for every layer and row of the session at once: k, v and n_src hold num_layers * rows
-  // values, layer by layer.
-  int import_prompt(int sid, const void* const* k, const void* const* v, const int64_t* n_src, int64_t n_tokens,
-                    hipStream_t stream);
+  // The same for every row of layers [layer0, layer0 + n_layers) at once: k, v and n_src hold
+  // n_layers * rows values, layer by layer.
+  int import_layers(int sid, int layer0, int n_layers, const void* const* k, const void* const* v,
+                    const int64_t* n_src, int64_t n_tokens, hipStream_t stream);
   // Read back tokens [0, n) of one (session, row, layer) into k, v [Hkv, n, D] (device).
   int export_tokens(int sid, int row, int layer, void* k, void* v, int64_t n_tokens, hipStream_t stream);
 

@@ -25,6 +25,10 @@ from . import _native as N
 nat = N.nat
 
 
+# Contiguous copies of a prompt's strided rows that are held for one import call, in bytes: enough
+# that the calls cost nothing beside the copies, and little beside the prompt's K/V.
+_MAX_HELD_COPIES = 64 << 20
+
 _LIVE_POOLS: "weakref.WeakSet[NativeKVPool]" = weakref.WeakSet()
 
 
@@ -162,32 +166,58 @@ class NativeKVPool:
                    n_tokens, self._stream())
 
     def import_prompt(self, sid: int, rows: int, keys, values, n_tokens: int) -> None:
-        """Every layer and row at once: keys[layer][row], values[layer][row] as for import_tokens."""
-        held = []  # the tensors the launches read
-        kp, vp, n_src = [], [], []
+        """Every layer and row: keys[layer][row], values[layer][row] as for import_tokens. One call, or
+        one per run of layers whose strided rows' copies stay within _MAX_HELD_COPIES."""
+        first, kp, vp, n_src = 0, [], [], []  # the open run: its first layer and its (layer, row) pairs
+        held, held_bytes = [], 0  # copies that the run's launches read
+
+        def flush(next_layer):
+            nonlocal first, held_bytes
+            n = len(kp)
+            if n:
+                self._call("import", self.lib.pgr_kv_import_layers, sid, first, n // rows, (ctypes.c_void_p * n)(*kp),
+                           (ctypes.c_void_p * n)(*vp), (ctypes.c_int64 * n)(*n_src), n_tokens, self._stream())
+            for args in (kp, vp, n_src, held):
+                args.clear()
+            first, held_bytes = next_layer, 0
+
+        hkv, d = self.num_kv_heads, self.head_dim
         for layer in range(self.num_layers):
             k, v = keys[layer], values[layer]
-            if (type(k) is torch.Tensor and type(v) is torch.Tensor and k.dim() == 4 and v.dim() == 4
-                    and k.shape[0] >= rows and v.shape[0] >= rows and k.shape[2] == v.shape[2]
-                    and k.is_contiguous() and v.is_contiguous()):
-                self._check_kv(k, v)  # rows of one contiguous tensor
-                self._check_heads(k.shape[1:])
-                self._check_heads(v.shape[1:])
-                ks, vs = k.stride(0) * k.element_size(), v.stride(0) * v.element_size()
-                k0, v0 = k.data_ptr(), v.data_ptr()
-                kp.extend(k0 + r * ks for r in range(rows))
-                vp.extend(v0 + r * vs for r in range(rows))
-                n_src.extend([k.shape[2]] * rows)
+            if type(k) is torch.Tensor and type(v) is torch.Tensor and k.is_contiguous() and v.is_contiguous():
+                sk, sv = k.shape, v.shape
+                if (len(sk) == len(sv) == 4 and sk[0] >= rows and sv[0] >= rows and sk[1] == sv[1] == hkv
+                        and sk[2] == sv[2] and sk[3] == sv[3] == d):  # rows of one contiguous tensor
+                    self._check_kv(k, v)
+                    stride = hkv * sk[2] * d * 2
+                    k0, v0 = k.data_ptr(), v.data_ptr()
+                    kp.extend(k0 + r * stride for r in range(rows))
+                    vp.extend(v0 + r * stride for r in range(rows))
+                    n_src.extend([sk[2]] * rows)
+                    continue
+            pairs = [(k[row], v[row]) for row in range(rows)]
+            nbytes = 0
+            for kr, vr in pairs:
+                cut = kr.shape != vr.shape
+                if cut or not kr.is_contiguous():
+                    nbytes += 2 * kr.numel()
+                if cut or not vr.is_contiguous():
+                    nbytes += 2 * vr.numel()
+            if held_bytes + nbytes > _MAX_HELD_COPIES:
+                flush(layer)
+            if nbytes > _MAX_HELD_COPIES:  # one layer's rows: one pair's copies alive at a time
+                for row, (kr, vr) in enumerate(pairs):
+                    self.import_tokens(sid, row, layer, kr, vr, n_tokens)
+                first = layer + 1
                 continue
-            for row in range(rows):
-                kr, vr = self._row_kv(k[row], v[row], n_tokens)
+            held_bytes += nbytes
+            for kr, vr in pairs:
+                kr, vr = self._row_kv(kr, vr, n_tokens)
                 held.append((kr, vr))
                 kp.append(kr.data_ptr())
                 vp.append(vr.data_ptr())
                 n_src.append(kr.shape[1])
-        n = len(kp)
-        self._call("import", self.lib.pgr_kv_import_prompt, sid, (ctypes.c_void_p * n)(*kp), (ctypes.c_void_p * n)(*vp),
-                   (ctypes.c_int64 * n)(*n_src), n_tokens, self._stream())
+        flush(self.num_layers)
 
     def export_tokens(self, sid: int, row: int, layer: int, n_tokens: int):
         k = torch.empty((self.num_kv_heads, n_tokens, self.head_dim), dtype=self.dtype, device=self.device)
@@ -218,17 +248,14 @@ class NativeKVPool:
         if k.dtype != self.dtype or v.dtype != self.dtype:
             raise TypeError(f"tensors must be {self.dtype}")
 
-    def _check_heads(self, shape: torch.Size) -> None:
-        """One row of a prompt: the kernel reads [Hkv, n_src, D] by this pool's Hkv and D."""
-        if len(shape) != 3 or shape[0] != self.num_kv_heads or shape[2] != self.head_dim:
-            raise ValueError(f"a row's keys and values must be [{self.num_kv_heads}, tokens, {self.head_dim}], "
-                             f"got {list(shape)}")
-
     def _row_kv(self, k: torch.Tensor, v: torch.Tensor, n_tokens: int) -> tuple[torch.Tensor, torch.Tensor]:
-        """One row's K and V as the import reads them: contiguous, of this pool's shape and of one length."""
+        """One row's K and V as the import reads them: contiguous, [Hkv, n_src, D] by this pool's Hkv
+        and D, and of one length."""
         self._check_kv(k, v)
-        self._check_heads(k.shape)
-        self._check_heads(v.shape)
+        for shape in (k.shape, v.shape):
+            if len(shape) != 3 or shape[0] != self.num_kv_heads or shape[2] != self.head_dim:
+                raise ValueError(f"a row's keys and values must be [{self.num_kv_heads}, tokens, {self.head_dim}], "
+                                 f"got {list(shape)}")
         if k.shape[1] != v.shape[1]:
             if min(k.shape[1], v.shape[1]) < n_tokens:
                 raise ValueError(f"keys of {k.shape[1]} and values of {v.shape[1]} tokens for {n_tokens}")

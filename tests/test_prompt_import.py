@@ -2,6 +2,8 @@
 pool's Hkv and D and one n_src for K and V, so a tensor of another shape is refused before a launch."""
 from __future__ import annotations
 
+import weakref
+
 import pytest
 import torch
 
@@ -67,7 +69,7 @@ def test_keys_and_values_of_two_lengths_share_one_stride(form, nk, nv):
     pool = _Pool()
     _import(pool, form, _kv(ROWS, HKV, nk, D), _kv(ROWS, HKV, nv, D))
     fn, args = pool.calls[-1]
-    n_src = args[5] if form == "single" else list(args[3])[-1]
+    n_src = args[5] if form == "single" else list(args[5])[-1]
     assert n_src == N  # both cut to the prompt's length
 
 
@@ -80,5 +82,32 @@ def test_one_length_beyond_the_prompt_is_read_in_place(form):
     if form == "single":
         assert args[3:6] == (k.data_ptr(), v.data_ptr(), N + 5)
     else:
-        assert list(args[1])[-1] == k[1].data_ptr() and list(args[2])[-1] == v[1].data_ptr()
-        assert list(args[3])[-2:] == [N + 5] * 2
+        assert args[:3] == (0, 0, LAYERS)  # session, first layer, layers
+        assert list(args[3])[-1] == k[1].data_ptr() and list(args[4])[-1] == v[1].data_ptr()
+        assert list(args[5])[-2:] == [N + 5] * 2
+
+
+@pytest.mark.parametrize("n,layers,spans", [
+    (16384, 8, [(0, 8)]),  # 4 MiB of copies per layer
+    (16384, 40, [(0, 16), (16, 16), (32, 8)]),
+    (524288, 2, ["row 0", "row 1", "row 0", "row 1"]),  # 128 MiB: a row's K and V at a time
+])
+def test_copies_of_a_strided_prompt_are_bounded(n, layers, spans):
+    strided = _kv(1, n, HKV, D).transpose(1, 2).expand(ROWS, HKV, n, D)
+    live, most = [], []
+
+    class Pool(_Pool):
+        def _row_kv(self, k, v, n_tokens):
+            got = super()._row_kv(k, v, n_tokens)
+            live.extend(weakref.ref(t) for t in got)
+            return got
+
+        def _call(self, what, fn, *args):
+            most.append(sum(t().numel() * 2 for t in live if t() is not None))
+            super()._call(what, fn, *args)
+
+    pool = Pool()
+    pool.num_layers = layers
+    pool.import_prompt(0, ROWS, [strided] * layers, [strided] * layers, n)
+    assert max(most) <= 64 << 20
+    assert [f"row {a[1]}" if fn == "pgr_kv_import" else a[1:3] for fn, a in pool.calls] == spans
