@@ -1240,6 +1240,9 @@ __global__ __launch_bounds__(kThreads) void paged_merge_kernel(const SeqInfo* __
   constexpr int kLanes = D / 2;          // threads per partial group (two dims each)
   constexpr int G = kThreads / kLanes;   // partial groups
   constexpr int kRed = kLanes < kWaveSize ? kLanes : kWaveSize;  // lanes of group 0 per wave
+  // Groups per round of the combine: all of them, but for the 128 of 1024 threads at head dim 16,
+  // whose LDS values in flight would not fit the 128 registers a thread has there.
+  constexpr int kCombine = G > 64 ? 16 : G;
   __shared__ float m_s[G], l_s[G];
   __shared__ float acc_s[G][D];
   __shared__ float dot_s[kLanes / kRed];
@@ -1378,14 +1381,14 @@ __global__ __launch_bounds__(kThreads) void paged_merge_kernel(const SeqInfo* __
     else
       x_cur = dot * (a.scale * kLog2e);
     float mf = x_cur;  // the current token is always valid: mf is finite
-#pragma unroll
+#pragma unroll kCombine
     for (int g2 = 0; g2 < G; ++g2) mf = fmaxf(mf, m_s[g2]);
     const float pc = __builtin_amdgcn_exp2f(x_cur - mf);
     const float pcr = Ty::to_f(Ty::cvt(pc));  // P rounded to the K/V type before P.V
     float lf = pc;
     float o0 = pcr * Ty::to_f((uint16_t)(vd & 0xffffu));
     float o1 = pcr * Ty::to_f((uint16_t)(vd >> 16));
-#pragma unroll
+#pragma unroll kCombine
     for (int g2 = 0; g2 < G; ++g2) {
       const float w = __builtin_amdgcn_exp2f(m_s[g2] - mf);  // empty group: m = -inf, w = 0
       lf += l_s[g2] * w;

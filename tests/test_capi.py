@@ -97,6 +97,15 @@ def test_workspace_covers_the_split_of_either_element_size():
     assert [slots(t, 64) for t in (256, 257)] == [1, 5]
 
 
+def test_no_kernel_spills_registers():
+    """Every kernel's metadata in the built library (a key, then its value as a msgpack integer): no
+    vector register spilled, no scratch memory."""
+    image = open(nat.LIB_PATH, "rb").read()
+    for key in (b".vgpr_spill_count", b".private_segment_fixed_size"):
+        values = [image[m.end()] for m in re.finditer(re.escape(key), image)]
+        assert len(values) >= 100 and not any(values), (key, len(values), [v for v in values if v])
+
+
 def test_missing_library_fails_loudly():
     code = (
         "import os, sys; os.environ['PGR_LIBRARY'] = '/nonexistent/libpgr.so'; "

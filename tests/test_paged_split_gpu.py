@@ -65,3 +65,16 @@ def test_uneven_sequences_with_windows_and_softcap():
     for _ in range(2):
         _, _, err = p.step(g, windows=[100, None], rounding_allowance=True)
         assert err < TOL
+
+
+def test_more_than_512_slots_at_head_dim_16():
+    """The merge's widest form: 1024 threads, 128 groups of slots combined in rounds."""
+    g = torch.Generator().manual_seed(16)
+    n = 33000  # 2063 blocks of 16 tokens, four per work item
+    p = Pair(layers=1, hq=2, hkv=1, d=16, tpb=16, dtype=torch.float16, pool_blocks=n // 16 + 8, host_blocks=n // 16 + 8)
+    p.add(ctx=n, capacity=n + 64, gen=g, vram_budget=(n // 16 + 4) * MIB16, ram_budget=1024 * MIB16, recent_window=1,
+          policy="sinks_heavy_hitter")
+    for _ in range(2):
+        res, ref, _ = p.step(g, rounding_allowance=True)
+        got, want = res[p.sids[0]]["block_attention"], ref["placement"][p.sids[0]]["scores"]
+        assert float(np.abs(np.array(got) - np.array(want)).max()) < 1e-5
