@@ -122,9 +122,11 @@ int pgr_attn_set_timing(int32_t on);
 int pgr_attn_kernel_time(double* ms, int64_t* launches, int64_t* bytes);
 /* No counterpart in the reference. For measurement: the attention (fold) launch of
  * pgr_attn_step, without its merge, over each of n_chunks chunks (k[c], v[c], all of one
- * shape, no masks, no running state: the merge is what reads and updates it), `reps` rounds,
- * back to back between one pair of fence-free events on `stream`; returns the mean
- * microseconds per launch and the K/V bytes each launch reads. The workspace is
+ * shape, no masks), `reps` rounds, back to back between one pair of fence-free events on
+ * `stream`; returns the mean microseconds per launch and the K/V bytes each launch reads. A
+ * chunk that one workgroup per head holds has no merge: its launches update a running state,
+ * here one in the workspace (fresh at the call's start, m, l and acc in the order and
+ * alignment of the partials). The workspace is
  * pgr_attn_step's (pgr_attn_workspace_bytes, fold mode). Synchronous; not under graph
  * capture. */
 int pgr_attn_bench_step(const void* q, const void* const* k, const void* const* v, int32_t n_chunks, int64_t batch,

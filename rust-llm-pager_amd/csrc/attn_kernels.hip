@@ -1737,7 +1737,7 @@ hipError_t launch_dense(int dtype, int mode, int d, const DenseLaunch& p, hipStr
   a.block_id_offset = p.block_id_offset;
   a.scale = p.scale;
   a.softcap = p.softcap;
-  const bool direct = p.n_split == 1 && !p.attention_only;
+  const bool direct = p.n_split == 1;
   a.m_state = direct ? p.m : nullptr;
   a.l_state = direct ? p.l : nullptr;
   a.acc_state = direct ? p.acc : nullptr;

@@ -311,16 +311,26 @@ int pgr_attn_bench_step(const void* q, const void* const* k, const void* const* 
     const DensePlan p =
         plan_dense(dtype, batch, num_query_heads, num_kv_heads, tokens, head_dim, PGR_MODE_FOLD, 16);
     if (workspace == nullptr || workspace_bytes < p.bytes) return set_err(pgr::kErrCapacity, "workspace too small");
+    pgr::DenseLaunch L =
+        dense_launch(p, q, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 16, batch,
+                     num_query_heads, num_kv_heads, tokens, scale, 0.f, workspace);
+    L.attention_only = true;
     hipEvent_t ev[2] = {nullptr, nullptr};
     hipError_t e = hipSuccess;
+    if (p.n_split == 1) {
+      // The fold launch updates the running state itself: a state in the place of the partials,
+      // which have its shape then. (Otherwise only the merge reads the state, and none is passed.)
+      L.m = L.pm;
+      L.l = L.pl;
+      L.acc = L.pacc;
+      e = pgr::launch_state_init(L.m, L.l, L.acc, batch * num_query_heads, head_dim, as_stream(stream));
+    }
     for (int i = 0; i < 2 && e == hipSuccess; ++i) e = hipEventCreateWithFlags(&ev[i], hipEventDisableSystemFence);
     if (e == hipSuccess) e = hipEventRecord(ev[0], as_stream(stream));
     for (int r = 0; r < reps && e == hipSuccess; ++r)
       for (int c = 0; c < n_chunks && e == hipSuccess; ++c) {
-        // The fold launch reads no running state (only the merge does), so none is passed.
-        pgr::DenseLaunch L = dense_launch(p, q, k[c], v[c], nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0,
-                                          16, batch, num_query_heads, num_kv_heads, tokens, scale, 0.f, workspace);
-        L.attention_only = true;
+        L.k = k[c];
+        L.v = v[c];
         e = pgr::launch_dense(dtype, PGR_MODE_FOLD, (int)head_dim, L, as_stream(stream));
       }
     if (e == hipSuccess) e = hipEventRecord(ev[1], as_stream(stream));

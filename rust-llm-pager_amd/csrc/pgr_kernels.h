@@ -46,7 +46,8 @@ struct DenseLaunch {
   // merge): the fold kernel's own duration for measurement.
   hipEvent_t ev_start = nullptr;
   hipEvent_t ev_stop = nullptr;
-  // Measurement only: launch the attention kernel and not the merge (m, l, acc untouched).
+  // Measurement only: launch the attention kernel and not the merge (m, l, acc untouched, unless
+  // there is one split: the attention kernel then updates them).
   bool attention_only = false;
 };
 

@@ -107,7 +107,7 @@ def test_back_to_back_attention_launches_keep_the_decode_intact():
 @pytest.mark.gpu
 def test_operator_fold_back_to_back_launches():
     """pgr_attn_bench_step: the operator's fold launches over several chunks back to back (no
-    merge, no running state); bytes per launch are the chunk's K+V; a workspace too small for
+    merge); bytes per launch are the chunk's K+V; a workspace too small for
     the chunk's partials is refused."""
     import ctypes
 
@@ -135,3 +135,35 @@ def test_operator_fold_back_to_back_launches():
         nat.check(lib.pgr_attn_bench_step(q.data_ptr(), karr, varr, 3, b, hq, hkv, tc, d, nat.DTYPE_F16, d**-0.5,
                                           ws.data_ptr(), 16, 1, ctypes.byref(us), ctypes.byref(nbytes), stream),
                   "bench_step")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tc", [64, 256])
+def test_operator_fold_back_to_back_launches_what_the_step_does(tc):
+    """A chunk in one workgroup per head is folded into the running state by the launch itself:
+    pgr_attn_bench_step's launches leave the state that as many pgr_attn_step calls do."""
+    import ctypes
+
+    import _pgr_native as nat
+    from pager_hf.streaming_attention import streaming_attention_state_init, streaming_attention_step
+
+    lib = nat.load()
+    hq, hkv, d, reps = 28, 4, 128, 2
+    g = torch.Generator().manual_seed(tc)
+    q = torch.randn(1, hq, d, generator=g).half().cuda()
+    chunks = [tuple(torch.randn(1, hkv, tc, d, generator=g).half().cuda() for _ in range(2)) for _ in range(3)]
+    ws_bytes = lib.pgr_attn_workspace_bytes(1, hq, hkv, tc, d, nat.MODE_FOLD, 16)
+    ws = torch.zeros(ws_bytes, dtype=torch.uint8, device="cuda")
+    karr = (ctypes.c_void_p * 3)(*[kc.data_ptr() for kc, _ in chunks])
+    varr = (ctypes.c_void_p * 3)(*[vc.data_ptr() for _, vc in chunks])
+    us, nbytes = ctypes.c_double(0), ctypes.c_int64(0)
+    nat.check(lib.pgr_attn_bench_step(q.data_ptr(), karr, varr, 3, 1, hq, hkv, tc, d, nat.DTYPE_F16, d**-0.5,
+                                      ws.data_ptr(), ws_bytes, reps, ctypes.byref(us), ctypes.byref(nbytes),
+                                      torch.cuda.current_stream().cuda_stream), "bench_step")
+    m, l, acc = streaming_attention_state_init(1, hq, d, q.device)
+    for _ in range(reps):
+        for kc, vc in chunks:
+            streaming_attention_step(q, kc, vc, m, l, acc)
+    floats = ws.view(torch.float32)
+    for got, want in ((floats[:hq], m), (floats[64:64 + hq], l), (floats[128:128 + hq * d], acc)):
+        assert torch.equal(got, want.flatten())
