@@ -45,9 +45,9 @@ const char* pgr_last_error(void);
  * Shapes follow pager_hf/streaming_attention.py: q [B, Hq, D]; k, v [B, Hkv, Tc, D]
  * contiguous; valid [B, Tc] int32 0/1 or NULL (all valid); active [B] int32 or NULL (all
  * active); online-softmax state m, l [B, Hq] and acc [B, Hq, D] fp32, updated in place.
- * q, k, v share one dtype: fp16, bf16 or fp32. D in {8, 16, 32, 64, 128, 256} (16-bit at
- * 32/64/128 runs on MFMA, the rest on a VALU kernel); Hq / Hkv <= 16; scale > 0; softcap <= 0
- * disables softcapping. Anything else returns PGR_ERR_UNSUPPORTED.
+ * q, k, v share one dtype: fp16, bf16 or fp32 (fp32 with fp32 products). D in {8, 16, 32, 64,
+ * 128, 256}; Hq / Hkv <= 16; scale > 0; softcap <= 0 disables softcapping. Anything else returns
+ * PGR_ERR_UNSUPPORTED.
  * `workspace` must hold pgr_attn_workspace_bytes(...) bytes of device memory.
  */
 #define PGR_MODE_FOLD 0
@@ -70,12 +70,14 @@ int pgr_attn_step(const void* q, const void* k, const void* v, const int32_t* va
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): the same
  * fold as pgr_attn_step, same kernels and results, with its split-K partials in a static
  * device array of the library (8 MiB per GPU, held until the process ends) instead of a
- * workspace. It calls no allocating routine. A chunk whose partials exceed 8 MiB is
- * rejected with PGR_ERR_CAPACITY. With fp16/bf16 q/k/v, chunks with batch * num_kv_heads
- * <= 496 always fit at head_dim <= 128 and n_rep <= 16. fp32 q/k/v count as more, smaller
- * partial slots: there chunks with batch * num_kv_heads <= 496 always fit while
- * head_dim * n_rep <= 1024 (head_dim 64 at n_rep 16, 128 at n_rep 8); at head_dim 128 with
- * n_rep 16 a long chunk of even one row is rejected (1 x 16 x 65536 x 128 counts as 8.5 MB).
+ * workspace. It calls no allocating routine. A chunk that counts as more than 8 MiB of
+ * partials is rejected with PGR_ERR_CAPACITY; the count belongs to this entry point's
+ * contract and may be more than the kernels use. With fp16/bf16 q/k/v, chunks with
+ * batch * num_kv_heads <= 496 always fit at head_dim <= 128 and n_rep <= 16. fp32 q/k/v count
+ * as more, smaller partial slots: there chunks with batch * num_kv_heads <= 496 always fit
+ * while head_dim * n_rep <= 1024 (head_dim 64 at n_rep 16, 128 at n_rep 8); at head_dim 128
+ * with n_rep 16 a long chunk of even one row is rejected (1 x 16 x 65536 x 128 counts as
+ * 8.5 MB).
  * Calls share their GPU's array. Outside graph capture the library orders them: a call on
  * another stream than the previous call's waits on the GPU (hipStreamWaitEvent) for the
  * previous call to finish, so calls from several streams or threads run one after another

@@ -362,8 +362,8 @@ int pgr_attn_step_noalloc(const void* q, const void* k, const void* v, const int
     // read and nothing needs clearing.
     const size_t need = noalloc_contract_bytes(batch, num_query_heads, num_kv_heads, tokens, head_dim, dtype);
     if (need > kNoAllocScratchBytes)
-      return set_err(pgr::kErrCapacity, "pgr_attn_step_noalloc: this chunk needs " + std::to_string(need) +
-                                            " bytes of split-K partials, more than the " +
+      return set_err(pgr::kErrCapacity, "pgr_attn_step_noalloc: this chunk counts as " + std::to_string(need) +
+                                            " bytes of split-K partials by the documented limit, more than the " +
                                             std::to_string(kNoAllocScratchBytes) +
                                             "-byte static scratch; use pgr_attn_step with a workspace");
     NoAllocDevice* dev = nullptr;

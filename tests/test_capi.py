@@ -97,6 +97,17 @@ def test_workspace_covers_the_split_of_either_element_size():
     assert [slots(t, 64) for t in (256, 257)] == [1, 5]
 
 
+def test_noalloc_limit_is_named_as_a_limit():
+    """A chunk that the kernels' own plan would hold, refused by the documented count (before any
+    GPU call): the message does not claim that the kernels need that much."""
+    lib = nat.load()
+    rc = lib.pgr_attn_step_noalloc(None, None, None, None, None, None, None, None, 1, 16, 1, 65536, 128,
+                                   nat.DTYPE_F32, 0.1, 0.0, None)
+    assert rc == nat.PGR_ERR_CAPACITY
+    assert lib.pgr_attn_workspace_bytes(1, 16, 1, 65536, 128, nat.MODE_FOLD, 16) < 8 << 20
+    assert "counts as" in nat.last_error() and "needs" not in nat.last_error()
+
+
 def test_no_kernel_spills_registers():
     """Every kernel's metadata in the built library (a key, then its value as a msgpack integer): no
     vector register spilled, no scratch memory."""

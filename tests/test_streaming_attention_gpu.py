@@ -454,7 +454,7 @@ def test_unsupported_head_dim_is_rejected():
 @pytest.mark.parametrize("b, hq, hkv, d, tokens, dtype", [
     (2, 28, 4, 128, 32768, torch.float16),    # 64 splits per (row, KV head), 4 merge groups
     (1, 14, 2, 64, 65536, torch.bfloat16),    # 256 splits, 8 groups: four batches of slots per group
-    (1, 8, 1, 256, 16384, torch.float16),     # head dim 256 (VALU kernel), 2 groups
+    (1, 8, 1, 256, 16384, torch.float16),     # head dim 256
     (1, 8, 2, 32, 8192, torch.float32),       # fp32 q/k/v
 ])
 def test_long_chunk_merges_many_split_slots(b, hq, hkv, d, tokens, dtype):

@@ -67,7 +67,7 @@ def _run(lib, noalloc, case, seed, masked):
 CASES = [
     ((8, 14, 2, 6000, 64, torch.float16), 1, True),
     ((2, 32, 8, 700, 128, torch.bfloat16), 2, False),
-    # fp32 q/k/v run the generic kernel, whose plan has more, smaller partial slots.
+    # fp32 q/k/v count as more, smaller partial slots.
     ((1, 16, 1, 32768, 128, torch.float32), 3, True),
     ((4, 8, 2, 3000, 64, torch.float32), 4, False),
 ]
@@ -85,7 +85,7 @@ def test_noalloc_matches_workspace_entry_point_on_consecutive_calls():
 
 @pytest.mark.parametrize("case", [
     (1200, 16, 1, 16, 128, torch.float16),  # 1,200 partial slots of 16 x 130 floats: ~10 MB
-    (1, 16, 1, 65536, 128, torch.float32),  # one row, but 1,024 slots of the generic kernel: ~8.5 MB
+    (1, 16, 1, 65536, 128, torch.float32),  # one row, but it counts as 1,024 slots: ~8.5 MB
 ])
 def test_noalloc_rejects_a_chunk_beyond_the_static_scratch(case):
     lib = nat.load()
