@@ -128,6 +128,16 @@ def test_missing_library_fails_loudly():
     assert "ImportError" in res.stdout, res.stdout + res.stderr
 
 
+def test_paged_path_imports_without_the_operator_call_path():
+    code = (
+        f"import sys; sys.path.insert(0, {os.path.join(ROOT, 'rust-llm-pager_amd')!r}); sys.modules['_pgr_ops'] = None\n"
+        "from pager_hf import PagedDecoder\n"
+        "try:\n    import pager_hf.streaming_attention\nexcept ImportError as e:\n    print('ImportError', e)\n"
+    )
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
+    assert res.returncode == 0 and "ImportError _pgr_ops.so is missing" in res.stdout, res.stdout + res.stderr
+
+
 def test_no_product_module_imports_the_oracle():
     pkg = os.path.join(ROOT, "rust-llm-pager_amd")
     offenders = []
