@@ -80,7 +80,7 @@ struct BF16 {
 // exchanges the odd rows of its first operand with the even rows of its second, and
 // v_permlane32_swap the halves: with x in both, the two results hold x of the two rows (halves)
 // of each pair. Two VALU moves where __shfl_xor is an LDS permute and a wait on the tile's
-// dependence chain; the same pairs are added in the same order.
+// dependence chain; the same pairs are added in the same order (times: paged_attn_kernel).
 // (The result's elements are read into scalars first: __builtin_bit_cast of a vector element
 // takes element 0.)
 __device__ __forceinline__ void row_pair(float x, float& a, float& b) {
@@ -439,9 +439,13 @@ struct DenseArgs {
 //
 // Below 64 dwords per lane and tile, two tiles per wave are in flight (double-buffered
 // registers). From 64 on (16-bit D 256, fp32 D 128) the tile is single-buffered in halves: the
-// next K is loaded under the softmax and P.V, the next V under the next scores. That needs half
-// the registers, so two waves per SIMD instead of one: 16.6 against 18.5 us at bf16 D 256, 28.1
-// against 27.7 at fp32 D 128. At fp32 D 256 (128 dwords) q comes from LDS as well.
+// next K is loaded under the softmax and P.V, the next V under the next scores. bf16 D 256 takes
+// 190 registers so, two waves per SIMD instead of one, and 16.6 against 18.5 us. fp32 D 128 takes
+// 160, three waves against two, and the forms tie in fold (32/8 heads, batch 8, 1000 / 4000 / 20000
+// tokens: 17.1 / 41.9 / 169 us single, 17.3 / 41.2 / 167 double); accumulate and the statistics pass
+// are 0.1-0.4 us faster single-buffered below 4000 tokens and slower on long chunks (20000 tokens:
+// 184 against 174, 133 against 113.5). At fp32 D 256 (128 dwords) q comes from LDS as well, and 254
+// registers and 36 accumulation registers still leave one wave per SIMD.
 template <class Ty, int D, int DR, int kMode>
 __global__ __launch_bounds__(256) void dense_attn_kernel(DenseArgs a) {
   using T = Tile<Ty, D>;
@@ -922,7 +926,8 @@ struct TileMeta {
 
 // Mass launches: units a work item's blocks hold at most (tiles, or whole blocks where that
 // would be more). (m, s) of 128 units take 16 KB of LDS; 64 at head dim 256, whose workgroup
-// merge takes 66 KB, so that two workgroups fit a CU.
+// merge takes 66 KB. (Registers decide how many workgroups a CU holds: two at head dim 128, 183
+// each, and one at 256, 256 and 12 accumulation registers.)
 template <int D>
 struct MassUnits {
   static constexpr int N = D == 256 ? 2 * kMaxWorkEntries : 4 * kMaxWorkEntries;
@@ -990,12 +995,14 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const WorkItem* __restr
   // most one and no wave holds the workgroup up by a whole block. With per-block mass (kMass)
   // a tile's (m, s) is one unit in LDS, and a block's units are combined after the loop; where
   // the blocks hold too many tiles for that, wave w folds whole blocks: entries w, w+4, ...
-  // (a unit is then a block). Against whole blocks dealt to the waves at every block size:
-  // 64 sequences at head dim 128 (32-token blocks) 23.15 -> 22.87 us per layer, 8 sequences up to
-  // 28770 tokens at head dim 64 23.0 -> 22.5, 4 of 32768 at head dim 128 99.9 -> 99.6. The cursor (fe, ftb) names the next fetch's entry and tile in
-  // block; the entry being fetched and the next one sit in SGPRs, and the one after is read
-  // (a scalar load) as a fetch is issued, a fetch ahead of its use. Entries past entry_count
-  // are never read by a fetch (the slots exist in every work item).
+  // (a unit is then a block). Us per layer with 32-token blocks, blocks dealt and lane sums by
+  // __shfl_xor / tiles dealt / row swaps (row_pair) / both: 64 sequences at head dim 128 23.15 /
+  // 23.10 / 23.06 / 22.87; 8 sequences up to 28770 tokens at head dim 64 23.0 / 22.75 / 22.7 / 22.5;
+  // 4 of 32768 at head dim 128 99.85 / 98.05 / 101.5 / 99.6: there the swaps lose what the dealing
+  // gains. The cursor (fe, ftb) names the next fetch's entry and tile in block; the entry being
+  // fetched and the next one sit in SGPRs, and the one after is read (a scalar load) as a fetch
+  // is issued, a fetch ahead of its use. Entries past entry_count are never read by a fetch (the
+  // slots exist in every work item).
   const bool by_tile = !kMass || tpb * kMaxWorkEntries <= kUnits;
   int fe = by_tile ? wave / tpb : wave, ftb = by_tile ? wave - (wave / tpb) * tpb : 0;
   const int step_e = by_tile ? kWaves / tpb : 0, step_tb = by_tile ? kWaves - step_e * tpb : 1;
@@ -1225,9 +1232,10 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(const WorkItem* __restr
 // thread in 256 threads: 64 sequences of 93 to 2038 tokens at head dim 128 (14 slots at most)
 // 25.6 -> 23.3 us, with block mass 27.2 -> 24.7; 8 sequences up to 28770 tokens at head dim 64
 // (74 slots) 20.0 -> 19.6, with block mass 22.25 -> 21.85; two of 16384 at 8/1 heads, head dim 256
-// (256 slots) 16.6 -> 15.2. (512 threads with 6 slots took 19.5 and 21.3 at the 8 sequences, but add
-// the slots in another order, which turns a 0.004 logit gap of the 8192-token TinyLlama run into
-// another token.)
+// (256 slots) 16.6 -> 15.2. 6 and 12 against the next of 8 and 16, head dim 64: 8 of 16384 (48
+// slots) 15.25 -> 15.13, 4 of 32768 (96 slots) 15.9 -> 15.55, with block mass 18.3 -> 18.0. (512
+// threads with 6 slots took 19.5 and 21.3 at the 8 uneven sequences, but add the slots in another
+// order, which turns a 0.004 logit gap of the 8192-token TinyLlama run into another token.)
 constexpr int kMergeBatch = 16;
 
 // The leading arguments are preloaded into SGPRs (as in paged_attn_kernel): the partial loads
@@ -1867,9 +1875,9 @@ hipError_t launch_mass_step_reduce(const SeqInfo* seqs, const int32_t* session_r
                                    hipStream_t stream) {
   if (n_sessions == 0 || max_blocks == 0 || num_layers == 0) return hipSuccess;
   dim3 grid((max_blocks + kStepMassBlocks - 1) / kStepMassBlocks, n_sessions);
-  mass_step_reduce_kernel<<<grid, kStepMassBlocks * kStepMassGroups, 0, stream>>>(seqs, session_rows, session_first, mass_w, layer_floats,
-                                                    num_layers, mass_accum, accum_stride, hq, mass_stride,
-                                                    max_blocks);
+  mass_step_reduce_kernel<<<grid, kStepMassBlocks * kStepMassGroups, 0, stream>>>(
+      seqs, session_rows, session_first, mass_w, layer_floats, num_layers, mass_accum, accum_stride, hq, mass_stride,
+      max_blocks);
   return hipGetLastError();
 }
 

@@ -209,7 +209,9 @@ bool ready(Py_ssize_t n, Py_ssize_t want) {
 }
 
 // A torch dispatch or function mode sees what the general path calls.
-bool modes_active() { return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled(); }
+bool modes_active() {
+  return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled();
+}
 
 // step(q, k, v, m, l, acc, valid, active, scale, softcap)
 PyObject* py_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -230,7 +232,8 @@ PyObject* py_stats(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!ready(n, 8)) return nullptr;
   return guarded([&]() -> PyObject* {
     Call c;
-    if (modes_active() || !prepare(c, a[0], a[1], nullptr, a[2], a[3], nullptr, a[4], a[5], a[6], a[7])) Py_RETURN_NONE;
+    if (modes_active() || !prepare(c, a[0], a[1], nullptr, a[2], a[3], nullptr, a[4], a[5], a[6], a[7]))
+      Py_RETURN_NONE;
     return run(c, kStats, 16, [&](void* ws, size_t bytes) {
       return g_stats(c.q, c.k, c.valid, c.active, c.m, c.l, c.b, c.hq,
                      c.hkv, c.tc, c.d, c.code, c.scale, c.softcap, ws, bytes, c.stream);
@@ -245,8 +248,8 @@ PyObject* py_accumulate(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     Call c;
     int64_t offset = 0, tpb = 0;
-    if (modes_active() || !prepare(c, a[0], a[1], a[2], a[3], a[4], a[5], a[9], a[10], a[11], a[12]) || !integer(a[7], &offset) ||
-        !integer(a[8], &tpb) || tpb <= 0)
+    if (modes_active() || !prepare(c, a[0], a[1], a[2], a[3], a[4], a[5], a[9], a[10], a[11], a[12]) ||
+        !integer(a[7], &offset) || !integer(a[8], &tpb) || tpb <= 0)
       Py_RETURN_NONE;
     const Tensor* mass = plain(a[6]);
     if (!mass || mass->scalar_type() != at::kFloat || mass->device() != c.dev || mass->dim() != 3 ||
