@@ -1695,7 +1695,7 @@ bool paged_head_dim_supported(int d) { return d == 16 || d == 32 || d == 64 || d
 
 bool dense_head_dim_supported(int d) { return d == 8 || paged_head_dim_supported(d); }
 
-int dense_wave_tokens(int dtype, int batch, int hkv, int tc, int d, int tokens_per_block, bool mass) {
+int dense_wave_tokens(int batch, int hkv, int tc, int d, int tokens_per_block, bool mass) {
   // Aim for about 2048 waves over the grid (8 per CU), each folding at least one 16-token tile.
   const long target = 2048;
   const long tiles = (tc + 15) / 16;
@@ -1703,16 +1703,12 @@ int dense_wave_tokens(int dtype, int batch, int hkv, int tc, int d, int tokens_p
   long per_wave = (tiles * rows + target - 1) / target;
   if (per_wave < 1) per_wave = 1;
   // A short chunk of a head stays in one workgroup, which then updates the state itself (one
-  // launch, no partials): up to 256 tokens and 64 KB of K. Back to back on the GPU, fold / stats /
-  // accumulate, split and merged -> one workgroup: 28/4 heads D 128 fp16, 256 tokens (64 KB) 7.2 /
+  // launch, no partials): up to 256 tokens and 32768 elements of K. Back to back on the GPU, fold /
+  // stats / accumulate, split and merged -> one workgroup: 28/4 heads D 128 fp16, 256 tokens 7.2 /
   // 6.1 / 6.4 -> 6.2 / 4.6 / 5.4 us, 512 tokens 7.2 / 6.2 / 6.6 -> 8.7 / 6.1 / 7.7; 8/1 D 256 bf16,
-  // 128 tokens (64 KB) 8.2 / 6.3 / 6.3 -> 7.5 / 4.3 / 6.3, 256 tokens 8.3 / 6.3 / 8.1 -> 9.6 / 6.0 /
-  // 8.5. fp32 reaches it at half the tokens: 28/4 D 128, 128 tokens (64 KB) 8.3 / 6.7 / 6.4 -> 7.5 /
-  // 5.0 / 6.4, 256 tokens (128 KB) 8.6 / 7.1 / 8.7 -> 10.1 / 6.9 / 9.1; 16/8 D 256 batch 2, 128
-  // tokens (128 KB) 12.3 / 9.4 / 13.0 -> 13.4 / 8.7 / 13.0; 32/4 D 64 batch 4, 256 tokens (64 KB)
-  // 7.2 / 6.2 / 6.9 -> 7.1 / 5.1 / 6.4. And a launch less on the host either way.
-  const long k_bytes = (long)tc * d * (dtype == kF32 ? 4 : 2);
-  if (tc <= 256 && k_bytes <= 65536 && per_wave * kWaves < tiles) per_wave = (tiles + kWaves - 1) / kWaves;
+  // 128 tokens 8.2 / 6.3 / 6.3 -> 7.5 / 4.3 / 6.3, 256 tokens 8.3 / 6.3 / 8.1 -> 9.6 / 6.0 / 8.5;
+  // and a launch less on the host either way.
+  if (tc <= 256 && (long)tc * d <= 32768 && per_wave * kWaves < tiles) per_wave = (tiles + kWaves - 1) / kWaves;
   long tokens = per_wave * 16;
   if (mass) {
     const long tpb = tokens_per_block;

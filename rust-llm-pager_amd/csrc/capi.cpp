@@ -3,7 +3,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cmath>
 #include <exception>
 #include <mutex>
@@ -59,13 +58,11 @@ struct DensePlan {
   size_t bytes = 0, o_pm = 0, o_pl = 0, o_pacc = 0;
 };
 
-DensePlan plan_dense(int dtype, int64_t batch, int64_t hq, int64_t hkv, int64_t tokens, int64_t d, int mode,
-                     int64_t tpb) {
+DensePlan plan_dense(int64_t batch, int64_t hq, int64_t hkv, int64_t tokens, int64_t d, int mode, int64_t tpb) {
   DensePlan p;
   if (tokens <= 0 || batch <= 0) return p;
   const bool mass = mode == PGR_MODE_ACCUMULATE;
-  p.wave_tokens =
-      pgr::dense_wave_tokens(dtype, (int)batch, (int)hkv, (int)tokens, (int)d, (int)(mass ? tpb : 16), mass);
+  p.wave_tokens = pgr::dense_wave_tokens((int)batch, (int)hkv, (int)tokens, (int)d, (int)(mass ? tpb : 16), mass);
   const int64_t per_wg = (int64_t)pgr::kWaves * p.wave_tokens;
   p.n_split = (int)((tokens + per_wg - 1) / per_wg);
   const size_t slots = (size_t)batch * hkv * p.n_split;
@@ -166,7 +163,7 @@ int run_dense(int mode, const void* q, const void* k, const void* v, const int32
   if (tokens == 0 || batch == 0) return pgr::kOk;  // nothing to fold: the state is unchanged
   if (!q || !k || !m || !l || (mode != PGR_MODE_STATS && (!v || !acc)))
     return set_err(pgr::kErrInvalid, "null tensor pointer");
-  const DensePlan p = plan_dense(dtype, batch, hq, hkv, tokens, d, mode, tpb);
+  const DensePlan p = plan_dense(batch, hq, hkv, tokens, d, mode, tpb);
   if (ws == nullptr || ws_bytes < p.bytes) return set_err(pgr::kErrCapacity, "workspace too small");
   pgr::DenseLaunch L = dense_launch(p, q, k, v, valid, active, m, l, acc, block_mass, max_blocks, block_id_offset, tpb,
                                     batch, hq, hkv, tokens, scale, softcap, ws);
@@ -272,12 +269,7 @@ size_t pgr_attn_workspace_bytes(int64_t batch, int64_t num_query_heads, int64_t 
   try {
     if (batch <= 0 || num_kv_heads <= 0 || num_query_heads <= 0 || tokens <= 0 || head_dim <= 0) return 0;
     if (mode == PGR_MODE_ACCUMULATE && (tokens_per_block <= 0 || tokens_per_block % 16 != 0)) return 0;
-    // The split follows the element size: the workspace covers both.
-    size_t bytes = 0;
-    for (int dtype : {pgr::kF16, pgr::kF32})
-      bytes = std::max(bytes, plan_dense(dtype, batch, num_query_heads, num_kv_heads, tokens, head_dim, mode,
-                                         tokens_per_block).bytes);
-    return bytes;
+    return plan_dense(batch, num_query_heads, num_kv_heads, tokens, head_dim, mode, tokens_per_block).bytes;
   } catch (...) {
     exception_status();
     return 0;
@@ -308,8 +300,7 @@ int pgr_attn_bench_step(const void* q, const void* const* k, const void* const* 
       return set_err(pgr::kErrInvalid, "pgr_attn_bench_step: inputs, chunks > 0, reps > 0 and outputs required");
     for (int c = 0; c < n_chunks; ++c)
       if (!k[c] || !v[c]) return set_err(pgr::kErrInvalid, "pgr_attn_bench_step: a null chunk");
-    const DensePlan p =
-        plan_dense(dtype, batch, num_query_heads, num_kv_heads, tokens, head_dim, PGR_MODE_FOLD, 16);
+    const DensePlan p = plan_dense(batch, num_query_heads, num_kv_heads, tokens, head_dim, PGR_MODE_FOLD, 16);
     if (workspace == nullptr || workspace_bytes < p.bytes) return set_err(pgr::kErrCapacity, "workspace too small");
     pgr::DenseLaunch L =
         dense_launch(p, q, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 16, batch,

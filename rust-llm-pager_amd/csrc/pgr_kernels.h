@@ -108,7 +108,7 @@ bool paged_head_dim_supported(int d);
 // Head dims of the dense operator kernels: 8, 16, 32, 64, 128, 256 (fp16, bf16 or fp32).
 bool dense_head_dim_supported(int d);
 // Dense launch geometry: consecutive tokens per wave (kWaves waves per workgroup).
-int dense_wave_tokens(int dtype, int batch, int hkv, int tc, int d, int tokens_per_block, bool mass);
+int dense_wave_tokens(int batch, int hkv, int tc, int d, int tokens_per_block, bool mass);
 
 hipError_t launch_dense(int dtype, int mode, int d, const DenseLaunch& p, hipStream_t stream);
 hipError_t launch_finalize(int dtype, const float* acc, const float* l, void* out, int rows, int d,

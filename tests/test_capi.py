@@ -81,22 +81,6 @@ def test_workspace_size_is_deterministic_and_positive():
     assert lib.pgr_attn_workspace_bytes(1, 14, 2, 0, 64, nat.MODE_FOLD, 16) == 0
 
 
-def test_workspace_covers_the_split_of_either_element_size():
-    """64 KB of K per head stay in one workgroup (one partial slot), so fp32 splits at half the
-    tokens; the size does not depend on the type and covers the larger."""
-    lib = nat.load()
-
-    def slots(tokens, d):  # of one head: m, l and acc
-        up = lambda n: (n + 255) // 256 * 256  # noqa: E731
-        sizes = {2 * up(4 * s) + up(4 * s * d): s for s in range(1, 9)}
-        return sizes[lib.pgr_attn_workspace_bytes(1, 1, 1, tokens, d, nat.MODE_FOLD, 16)]
-
-    # fp32 at head dim 256 and 128: one slot up to 64 KB, a slot per 64 tokens beyond.
-    assert [slots(t, 256) for t in (64, 65, 128, 256)] == [1, 2, 2, 4]
-    assert [slots(t, 128) for t in (128, 129, 256)] == [1, 3, 4]
-    assert [slots(t, 64) for t in (256, 257)] == [1, 5]
-
-
 def test_noalloc_limit_is_named_as_a_limit():
     """A chunk that the kernels' own plan would hold, refused by the documented count (before any
     GPU call): the message does not claim that the kernels need that much."""
