@@ -1706,8 +1706,12 @@ int dense_wave_tokens(int batch, int hkv, int tc, int d, int tokens_per_block, b
   // launch, no partials): up to 256 tokens and 32768 elements of K. Back to back on the GPU, fold /
   // stats / accumulate, split and merged -> one workgroup: 28/4 heads D 128 fp16, 256 tokens 7.2 /
   // 6.1 / 6.4 -> 6.2 / 4.6 / 5.4 us, 512 tokens 7.2 / 6.2 / 6.6 -> 8.7 / 6.1 / 7.7; 8/1 D 256 bf16,
-  // 128 tokens 8.2 / 6.3 / 6.3 -> 7.5 / 4.3 / 6.3, 256 tokens 8.3 / 6.3 / 8.1 -> 9.6 / 6.0 / 8.5;
-  // and a launch less on the host either way.
+  // 128 tokens 8.2 / 6.3 / 6.3 -> 7.5 / 4.3 / 6.3, 256 tokens 8.3 / 6.3 / 8.1 -> 9.6 / 6.0 / 8.5.
+  // fp32 at the line holds twice the bytes, and its fold takes longer than split: 28/4 D 128, 256
+  // tokens 8.6 / 7.1 / 8.7 -> 10.1 / 6.9 / 9.1; 16/8 D 256 batch 2, 128 tokens 12.3 / 9.4 / 13.0 ->
+  // 13.4 / 8.7 / 13.0. But calls of this size are host-bound, and a launch less is worth more: state
+  // init, fold and finalize from Python 19.7 -> 16.4 and 19.1 -> 17.2 us, a two-pass run 26.8 ->
+  // 20.8 and 25.7 -> 24.6. So the line is the same number of elements for every type.
   if (tc <= 256 && (long)tc * d <= 32768 && per_wave * kWaves < tiles) per_wave = (tiles + kWaves - 1) / kWaves;
   long tokens = per_wave * 16;
   if (mass) {

@@ -31,7 +31,7 @@ CHUNKS = [[64, 65, 128, 129], [256, 257, 1, 480], [1024, 16], [2600, 3], [5001, 
 @pytest.mark.parametrize("chunks", CHUNKS, ids=lambda c: "+".join(map(str, c)))
 @pytest.mark.parametrize("hq,hkv,d,dtype", [
     (7, 1, 64, torch.float16), (16, 1, 128, torch.bfloat16), (6, 3, 8, torch.float16), (4, 2, 256, torch.bfloat16),
-    (4, 2, 256, torch.float32), (5, 1, 32, torch.float32), (4, 4, 16, torch.float16),
+    (4, 2, 256, torch.float32), (4, 2, 128, torch.float32), (5, 1, 32, torch.float32), (4, 4, 16, torch.float16),
 ])
 def test_chunks_on_both_sides_of_the_split(hq, hkv, d, dtype, chunks):
     print(f"operator split: {hq}/{hkv} d={d} {dtype} {chunks}", flush=True)
