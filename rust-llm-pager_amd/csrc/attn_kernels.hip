@@ -446,7 +446,15 @@ struct DenseArgs {
 // are 0.1-0.4 us faster single-buffered below 4000 tokens and slower on long chunks (20000 tokens:
 // 184 against 174, 133 against 113.5). At fp32 D 256 (128 dwords) q comes from LDS as well, and 254
 // registers and 36 accumulation registers still leave one wave per SIMD.
-template <class Ty, int D, int DR, int kMode>
+//
+// kTileMax (16-bit fold at head dims 32 to 128, a head's whole chunk in one workgroup, several
+// tiles per wave): a tile's weights are taken, and rounded for P.V, under the tile's own maximum,
+// and its sums scaled to the running one. The same chunk split over workgroups has one tile per
+// wave, whose largest weight is an exact 1; under one running maximum per wave acc was up to 1.13
+// times, and the output 1.04 times, as far from 64 bits at 130 and 200 tokens. Now both are as
+// split, for 0.05-0.4 us of the launch (28/4 heads, D 128, 256 tokens 6.2 -> 6.5). (The kernel that
+// head dims 8, 16 and 256 had before took 64 tokens under one maximum: no loss there.)
+template <class Ty, int D, int DR, int kMode, bool kTileMax = false>
 __global__ __launch_bounds__(256) void dense_attn_kernel(DenseArgs a) {
   using T = Tile<Ty, D>;
   constexpr bool kFold = (kMode == kModeFold || kMode == kModeStats);
@@ -561,7 +569,21 @@ __global__ __launch_bounds__(256) void dense_attn_kernel(DenseArgs a) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) s[i] = ok[i] ? transform_score(s4[i], a.scale, a.softcap) : kNegInf;
 
-    if constexpr (kFold) {
+    if constexpr (kTileMax) {
+      const float tmax = wave_max_g(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])));
+      const float m_new = fmaxf(m_run, tmax);
+      const bool none = (tmax == kNegInf);  // nothing valid in the tile
+      const float alpha = m_new == kNegInf ? 0.f : __expf(m_run - m_new);
+      const float beta = none ? 0.f : __expf(tmax - m_new);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[i] = none ? 0.f : __expf(s[i] - tmax);
+      l_run = l_run * alpha + ((p[0] + p[1]) + (p[2] + p[3])) * beta;
+      const u32x2 pb = {Ty::pack(p[0], p[1]), Ty::pack(p[2], p[3])};
+#pragma unroll
+      for (int j = 0; j < D / 16; ++j)
+        acc[j] = acc[j] * alpha + Ty::mma(v_tile(t.v, j), pb, f32x4{0.f, 0.f, 0.f, 0.f}) * beta;
+      m_run = m_new;
+    } else if constexpr (kFold) {
       const float tmax = wave_max_g(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])));
       const float m_new = fmaxf(m_run, tmax);
       const bool empty = (m_new == kNegInf);
@@ -1576,6 +1598,12 @@ hipError_t launch_dense_merge(const DenseArgs& a, int mode, int batch, int d, fl
 template <class Ty, int D, int DR>
 hipError_t launch_dense_t(const DenseArgs& a, int mode, int batch, hipStream_t stream) {
   dim3 grid(a.n_split, a.hkv, batch);
+  if constexpr (!std::is_same<Ty, F32>::value && D >= 32 && D <= 128) {
+    if (mode == kModeFold && a.m_state != nullptr && a.wave_tokens > 16) {
+      dense_attn_kernel<Ty, D, DR, kModeFold, true><<<grid, 256, 0, stream>>>(a);
+      return hipGetLastError();
+    }
+  }
   switch (mode) {
     case kModeFold:
       dense_attn_kernel<Ty, D, DR, kModeFold><<<grid, 256, 0, stream>>>(a);
@@ -1705,7 +1733,7 @@ int dense_wave_tokens(int batch, int hkv, int tc, int d, int tokens_per_block, b
   // A short chunk of a head stays in one workgroup, which then updates the state itself (one
   // launch, no partials): up to 256 tokens and 32768 elements of K. Back to back on the GPU, fold /
   // stats / accumulate, split and merged -> one workgroup: 28/4 heads D 128 fp16, 256 tokens 7.2 /
-  // 6.1 / 6.4 -> 6.2 / 4.6 / 5.4 us, 512 tokens 7.2 / 6.2 / 6.6 -> 8.7 / 6.1 / 7.7; 8/1 D 256 bf16,
+  // 6.1 / 6.4 -> 6.5 / 4.6 / 5.4 us, 512 tokens 7.2 / 6.2 / 6.6 -> 8.7 / 6.1 / 7.7; 8/1 D 256 bf16,
   // 128 tokens 8.2 / 6.3 / 6.3 -> 7.5 / 4.3 / 6.3, 256 tokens 8.3 / 6.3 / 8.1 -> 9.6 / 6.0 / 8.5.
   // fp32 at the line holds twice the bytes, and its fold takes longer than split: 28/4 D 128, 256
   // tokens 8.6 / 7.1 / 8.7 -> 10.1 / 6.9 / 9.1; 16/8 D 256 batch 2, 128 tokens 12.3 / 9.4 / 13.0 ->

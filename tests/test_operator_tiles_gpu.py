@@ -151,3 +151,24 @@ def test_fp32_sums_at_small_head_dims(hq, hkv, d, bound):
     mean = sum(errors) / len(errors)
     print(f"fp32 sums, head dim {d}: {mean:.3e}", flush=True)
     assert mean <= bound
+
+
+@pytest.mark.parametrize("dtype,bound", [(torch.float16, 1.49e-4), (torch.bfloat16, 1.19e-3)], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("hq,hkv,d", [(16, 1, 32), (32, 4, 64), (28, 4, 128)])
+def test_16_bit_weights_of_short_chunks(hq, hkv, d, dtype, bound):
+    """The relative error of acc (2-norm, mean over 4 inputs) at 200 tokens in one workgroup, four
+    tiles per wave: from rounding the weights before P.V, so from the maximum they are taken under.
+    Bounds: half way between a maximum per tile, as split over workgroups (1.38 to 1.41e-4 in fp16,
+    1.10 to 1.12e-3 in bf16) and one per wave (1.56 to 1.58e-4 and 1.25 to 1.27e-3)."""
+    errors = []
+    for seed in range(4):
+        q, k, v, valid = _inputs((16, hq, hkv, 200), d, dtype, 100 * d + seed)
+        valid.fill_(1)
+        _, l_ref, out_ref, _ = _reference(q, k, v, valid)
+        m, l, acc = streaming_attention_state_init(16, hq, d, torch.device("cuda"))
+        streaming_attention_step(q.cuda(), k.cuda(), v.cuda(), m, l, acc)
+        want = out_ref * l_ref[..., None]
+        errors.append(float((acc.cpu().double() - want).norm() / want.norm()))
+    mean = sum(errors) / len(errors)
+    print(f"{dtype} weights, head dim {d}: {mean:.3e}", flush=True)
+    assert mean <= bound
